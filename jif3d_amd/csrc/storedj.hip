@@ -52,12 +52,24 @@ constexpr int kColPad = 256;   // J column count multiple (one J^T R workgroup)
 constexpr int kChunk = 16;     // cells per pipeline chunk of J M
 constexpr int kStage = 32;     // rows per LDS stage of J^T R
 constexpr int kPitch = 257;    // LDS row pitch (floats) of the J^T R stage
+typedef float f32x2 __attribute__((ext_vector_type(2)));
 typedef float f32x4 __attribute__((ext_vector_type(4)));
 typedef float f32x16 __attribute__((ext_vector_type(16)));
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 
 inline unsigned blocks_for(long n) { return (unsigned)((n + kBlock - 1) / kBlock); }
 inline long round_up(long v, long m) { return (v + m - 1) / m * m; }
+
+// Padded right-hand-side count of a product: a multiple of 64 (the products' tile), or one
+// narrow tile when it holds them all: 32 right-hand sides in FP32, 16 in FP64.  A cached
+// data or gradient evaluation of an inversion has one; with the full tile it was bound by
+// matrix-core work on zeros, with the narrow one by the read of J.  Every right-hand side's
+// sums keep their order, so the results are the same bits for every width.
+inline int rhs_pad(int gemm_precision, bool fp64, long nrhs) {
+  if (fp64 && nrhs <= 16) return 16;
+  if (!fp64 && gemm_precision == JGM_GEMM_FP32 && nrhs <= 32) return 32;
+  return (int)round_up(nrhs, 64);
+}
 
 __host__ __device__ inline int compact_rows(int kind) {
   switch (kind) {
@@ -202,21 +214,22 @@ __device__ __forceinline__ void to_bf16(const float (&x)[8], bf16x8& hi, bf16x8&
   }
 }
 
-// acc[ta][tb] += A_ta B_tb for a 2 x 2 block of 32x32 tiles.  Element s of a lane's
+// acc[ta][tb] += A_ta B_tb for an NA x NB block of 32x32 tiles.  Element s of a lane's
 // operands is k-step s (FP32: the lane's k is lane/32 within each step) or, for BF16,
 // element s of the single 16-deep step (k = 8 * (lane/32) + s); A and B elements with
 // the same index always refer to the same k.
-template <int PREC>
-__device__ __forceinline__ void mma_block(const float (&a)[2][8], const float (&b)[2][8],
-                                          f32x16 (&acc)[2][2]) {
+template <int PREC, int NA, int NB>
+__device__ __forceinline__ void mma_block(const float (&a)[NA][8], const float (&b)[NB][8],
+                                          f32x16 (&acc)[NA][NB]) {
   if constexpr (PREC == JGM_GEMM_FP32) {
 #pragma unroll
     for (int s = 0; s < 8; ++s)
 #pragma unroll
-      for (int ta = 0; ta < 2; ++ta)
+      for (int ta = 0; ta < NA; ++ta)
 #pragma unroll
-        for (int tb = 0; tb < 2; ++tb) acc[ta][tb] = mfma32(a[ta][s], b[tb][s], acc[ta][tb]);
+        for (int tb = 0; tb < NB; ++tb) acc[ta][tb] = mfma32(a[ta][s], b[tb][s], acc[ta][tb]);
   } else {
+    static_assert(NA == 2 && NB == 2, "narrow tiles: FP32 only");
     constexpr bool R = PREC == JGM_GEMM_BF16_REFINED;
     bf16x8 ah[2], al[2], bh[2], bl[2];
 #pragma unroll
@@ -240,11 +253,12 @@ __device__ __forceinline__ void mma_block(const float (&a)[2][8], const float (&
 // Two-level accumulation: the MFMA accumulators are added into FP32 totals and reset
 // every 256 k, so no FP32 running sum grows longer than 256 k (the error of one long
 // FP32 sum grows with its length).
-__device__ __forceinline__ void flush(f32x16 (&acc)[2][2], float (&tot)[2][2][16]) {
+template <int NA, int NB>
+__device__ __forceinline__ void flush(f32x16 (&acc)[NA][NB], float (&tot)[NA][NB][16]) {
 #pragma unroll
-  for (int ta = 0; ta < 2; ++ta)
+  for (int ta = 0; ta < NA; ++ta)
 #pragma unroll
-    for (int tb = 0; tb < 2; ++tb)
+    for (int tb = 0; tb < NB; ++tb)
 #pragma unroll
       for (int r = 0; r < 16; ++r) {
         tot[ta][tb][r] += acc[ta][tb][r];
@@ -272,13 +286,15 @@ __device__ __forceinline__ void xcd_item(int w, int nw, int row_tiles, int& spli
 // Y partials: Yp[split][row][P].  Grid: x = nsplit * row_tiles workgroups in XCD order
 // (xcd_item), y = right-hand-side tiles of 64.  Each split covers `per` cells (a
 // multiple of 64).
+template <int NT>
 struct JmFrag {
-  float a[2][8], b[2][8];
+  float a[2][8], b[NT][8];
 };
 // register stages of k_gemm_jm: 4 (234 VGPRs for FP32, no spills) reads FP32 J at 113
 // TFLOP/s on 7168 x 131072 with the clocks up; 2 reaches 84, 3 97; 5 and 6 need AGPR
-// copies and are slower
-constexpr int kJmStages = 4;
+// copies and are slower.  One right-hand-side tile leaves registers for 6.
+template <int NT>
+constexpr int kJmStages = NT == 1 ? 6 : 4;
 typedef unsigned u32x4 __attribute__((ext_vector_type(4)));
 
 // The BF16-refined product may take M already split (MPRE: its high and low BF16 parts Mh,
@@ -289,7 +305,7 @@ struct JmFragPre {
   bf16x8 bh[2], bl[2];
 };
 
-template <int PREC, bool MPRE = false>
+template <int PREC, bool MPRE = false, int NT = 2>
 __global__ __launch_bounds__(kBlock) void k_gemm_jm(const float* __restrict__ J, long ld, long R,
                                                     long colpad, const float* __restrict__ Mt,
                                                     const bf16x8* __restrict__ Mh,
@@ -297,6 +313,8 @@ __global__ __launch_bounds__(kBlock) void k_gemm_jm(const float* __restrict__ J,
                                                     int row_tiles, int nsplit,
                                                     float* __restrict__ Yp) {
   static_assert(!MPRE || PREC == JGM_GEMM_BF16_REFINED, "split M: the refined product only");
+  static_assert(NT == 2 || (NT == 1 && PREC == JGM_GEMM_FP32), "narrow tiles: FP32 only");
+  constexpr int NS = kJmStages<NT>;
   const int w = blockIdx.x;
   int split, rt;
   xcd_item(w, nsplit * row_tiles, row_tiles, split, rt);
@@ -305,40 +323,41 @@ __global__ __launch_bounds__(kBlock) void k_gemm_jm(const float* __restrict__ J,
   const int li = lane & 31, lk = lane >> 5;
   const long row0 = (long)rt * 256 + wave * 64;
   if (row0 >= ld) return;  // whole wave outside the padded rows; no barriers follow
-  const int b0 = blockIdx.y * 64;
+  const int b0 = blockIdx.y * 32 * NT;
   const long c0 = (long)split * per;
   const long cend = c0 + per < colpad ? c0 + per : colpad;
   const int nchunk = cend > c0 ? (int)((cend - c0) / kChunk) : 0;
-  const float* Jw = J + row0 + li;
+  const float* Jw = J + row0 + 2 * li;
   const float* Mw = Mt + b0 + li;
-  f32x16 acc[2][2];
+  f32x16 acc[2][NT];
 #pragma unroll
   for (int ta = 0; ta < 2; ++ta)
 #pragma unroll
-    for (int tb = 0; tb < 2; ++tb)
+    for (int tb = 0; tb < NT; ++tb)
 #pragma unroll
       for (int r = 0; r < 16; ++r) acc[ta][tb][r] = 0.0f;
-  float tot[2][2][16];
+  float tot[2][NT][16];
 #pragma unroll
   for (int ta = 0; ta < 2; ++ta)
 #pragma unroll
-    for (int tb = 0; tb < 2; ++tb)
+    for (int tb = 0; tb < NT; ++tb)
 #pragma unroll
       for (int r = 0; r < 16; ++r) tot[ta][tb][r] = 0.0f;
-  // a ring of kJmStages chunks in registers: chunk q is loaded while q - kJmStages + 1 is
-  // multiplied, so kJmStages - 1 chunks of loads are in flight behind each MFMA block
-  using Frag = std::conditional_t<MPRE, JmFragPre, JmFrag>;
-  Frag f[kJmStages];
+  // a ring of NS chunks in registers: chunk q is loaded while q - NS + 1 is
+  // multiplied, so NS - 1 chunks of loads are in flight behind each MFMA block
+  using Frag = std::conditional_t<MPRE, JmFragPre, JmFrag<NT>>;
+  Frag f[NS];
   auto load = [&](Frag& g, int q) {
     const long cb = c0 + (long)(q < nchunk ? q : nchunk - 1) * kChunk;  // past the end: unused
 #pragma unroll
     for (int s = 0; s < 8; ++s) {
       const long cell = cb + chunk_k<PREC>(s, lk);
-      g.a[0][s] = __builtin_nontemporal_load(Jw + cell * ld);
-      g.a[1][s] = __builtin_nontemporal_load(Jw + cell * ld + 32);
+      const f32x2 v = __builtin_nontemporal_load((const f32x2*)(Jw + cell * ld));
+      g.a[0][s] = v[0];
+      g.a[1][s] = v[1];
       if constexpr (!MPRE) {
-        g.b[0][s] = Mw[cell * P];
-        g.b[1][s] = Mw[cell * P + 32];
+#pragma unroll
+        for (int t = 0; t < NT; ++t) g.b[t][s] = Mw[cell * P + 32 * t];
       }
     }
     if constexpr (MPRE) {
@@ -356,11 +375,11 @@ __global__ __launch_bounds__(kBlock) void k_gemm_jm(const float* __restrict__ J,
   // which would expose the full memory latency once per chunk
   if (nchunk > 0) {
 #pragma unroll
-    for (int d = 0; d < kJmStages - 1; ++d) load(f[d], d);
-    for (int q = 0; q < nchunk; q += kJmStages) {
+    for (int d = 0; d < NS - 1; ++d) load(f[d], d);
+    for (int q = 0; q < nchunk; q += NS) {
 #pragma unroll
-      for (int d = 0; d < kJmStages; ++d) {
-        load(f[(d + kJmStages - 1) % kJmStages], q + d + kJmStages - 1);
+      for (int d = 0; d < NS; ++d) {
+        load(f[(d + NS - 1) % NS], q + d + NS - 1);
         __builtin_amdgcn_sched_barrier(0);
         if (q + d < nchunk) {
           if constexpr (MPRE) {
@@ -386,16 +405,17 @@ __global__ __launch_bounds__(kBlock) void k_gemm_jm(const float* __restrict__ J,
     }
   }
   flush(acc, tot);
-  // D layout of a 32x32 MFMA: register r of lane l holds (row 8*(r/4) + 4*(l/32) + r%4, col l%32)
+  // D layout of a 32x32 MFMA: register r of lane l holds (row 8*(r/4) + 4*(l/32) + r%4, col
+  // l%32); row i of tile ta is the wave's row 2 i + ta
   float* out = Yp + (long)split * R * P;
 #pragma unroll
   for (int ta = 0; ta < 2; ++ta)
 #pragma unroll
     for (int r = 0; r < 16; ++r) {
-      const long row = row0 + 32 * ta + 8 * (r >> 2) + 4 * lk + (r & 3);
+      const long row = row0 + 2 * (8 * (r >> 2) + 4 * lk + (r & 3)) + ta;
       if (row < R) {
-        out[row * P + b0 + li] = tot[ta][0][r];
-        out[row * P + b0 + 32 + li] = tot[ta][1][r];
+#pragma unroll
+        for (int t = 0; t < NT; ++t) out[row * P + b0 + 32 * t + li] = tot[ta][t][r];
       }
     }
 }
@@ -735,26 +755,28 @@ __global__ __launch_bounds__(kBlock) void k_gemm_jm_reduce(const float* __restri
 // [k / 8][P] layout of k_rows_to_bf16_hilo; a stage holds them in the R area of LDS as
 // [group][rhs] (high parts, then low parts), a lane's A operand for a tile is one 16-byte
 // read of each, and only J is split in registers; the same values and MFMA order.
-template <int PREC, bool MPRE = false>
+template <int PREC, bool MPRE = false, int NT = 2>
 __global__ __launch_bounds__(kBlock) void k_gemm_jtr(const float* __restrict__ J, long ld, long N,
                                                      long nblk, const float* __restrict__ Rt,
                                                      const bf16x8* __restrict__ Rhi,
                                                      const bf16x8* __restrict__ Rlo, int P,
                                                      float* __restrict__ G, long ldg, int nrhs) {
   static_assert(!MPRE || PREC == JGM_GEMM_BF16_REFINED, "split R: the refined product only");
+  static_assert(NT == 2 || (NT == 1 && PREC == JGM_GEMM_FP32), "narrow tiles: FP32 only");
+  constexpr int W = 32 * NT;  // right-hand sides of a workgroup
   static_assert(kStage * 64 * sizeof(float) == 2 * (kStage / 8) * 64 * sizeof(bf16x8),
                 "the split R stage fills the R area");
   __shared__ float jt[kStage * kPitch];                           // [row][cell]
-  __shared__ __attribute__((aligned(16))) float rt[kStage * 64];  // [row][rhs]
+  __shared__ __attribute__((aligned(16))) float rt[kStage * W];   // [row][rhs]
   bf16x8* const rth = reinterpret_cast<bf16x8*>(rt);              // MPRE: [group][rhs]
   bf16x8* const rtl = rth + (kStage / 8) * 64;
-  const int b0 = blockIdx.y * 64;
+  const int b0 = blockIdx.y * W;
   const int tid = threadIdx.x;
   const int wave = tid >> 6, lane = tid & 63;
   const int li = lane & 31, lk = lane >> 5;
-  // loaders: J by 16-byte pieces (8 per cell line), Rt by 16-byte pieces (16 per row)
+  // loaders: J by 16-byte pieces (8 per cell line), Rt by 16-byte pieces (8 NT per row)
   const int jpart = tid & 7, jcell = tid >> 3;
-  const int rpart = tid & 15, rrow = tid >> 4;
+  const int rpart = tid & (8 * NT - 1), rrow = tid / (8 * NT);
   const float* Rl = Rt + (long)rrow * P + b0 + rpart * 4;
   const long nst = ld / kStage;
   for (long blk = blockIdx.x; blk < nblk; blk += gridDim.x) {
@@ -764,8 +786,8 @@ __global__ __launch_bounds__(kBlock) void k_gemm_jtr(const float* __restrict__ J
     // and p1 hold the next two stages' pieces.  Measured against one stage on the same
     // GPU, J 7168 x 131072, 64 right-hand sides: FP32 1.23 -> 1.19 ms, BF16 0.72 -> 0.67 ms,
     // BF16-refined 0.83 -> 0.81 ms.
-    f32x4 pj0[8], pr0[2], pj1[8], pr1[2];
-    auto gload = [&](long st, f32x4 (&pj)[8], f32x4 (&pr)[2]) {
+    f32x4 pj0[8], pr0[NT], pj1[8], pr1[NT];
+    auto gload = [&](long st, f32x4 (&pj)[8], f32x4 (&pr)[NT]) {
       const long r0 = (st < nst ? st : nst - 1) * kStage;  // past the end: unused reload
 #pragma unroll
       for (int q = 0; q < 8; ++q)
@@ -778,19 +800,19 @@ __global__ __launch_bounds__(kBlock) void k_gemm_jtr(const float* __restrict__ J
         pr[1] = __builtin_bit_cast(f32x4, Rlo[gi]);
       } else {
 #pragma unroll
-        for (int h = 0; h < 2; ++h) pr[h] = *(const f32x4*)(Rl + (r0 + 16 * h) * P);
+        for (int h = 0; h < NT; ++h) pr[h] = *(const f32x4*)(Rl + (r0 + 16 * h) * P);
       }
     };
-    f32x16 acc[2][2];  // [rhs tile][cell tile]
-    float tot[2][2][16];
+    f32x16 acc[NT][2];  // [rhs tile][cell tile]
+    float tot[NT][2][16];
 #pragma unroll
-    for (int ta = 0; ta < 2; ++ta)
+    for (int ta = 0; ta < NT; ++ta)
 #pragma unroll
       for (int tb = 0; tb < 2; ++tb)
 #pragma unroll
         for (int r = 0; r < 16; ++r) acc[ta][tb][r] = tot[ta][tb][r] = 0.0f;
     // stage st: to LDS from (pj, pr), refill (pj, pr) with stage st + 2, multiply
-    auto stage = [&](long st, f32x4 (&pj)[8], f32x4 (&pr)[2]) {
+    auto stage = [&](long st, f32x4 (&pj)[8], f32x4 (&pr)[NT]) {
       __syncthreads();  // the previous stage has been consumed
 #pragma unroll
       for (int q = 0; q < 8; ++q) {
@@ -805,20 +827,20 @@ __global__ __launch_bounds__(kBlock) void k_gemm_jtr(const float* __restrict__ J
         rtl[tid] = __builtin_bit_cast(bf16x8, pr[1]);
       } else {
 #pragma unroll
-        for (int h = 0; h < 2; ++h) *(f32x4*)(rt + (rrow + 16 * h) * 64 + rpart * 4) = pr[h];
+        for (int h = 0; h < NT; ++h) *(f32x4*)(rt + (rrow + 16 * h) * W + rpart * 4) = pr[h];
       }
       __syncthreads();
       gload(st + 2, pj, pr);
       __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
       for (int half = 0; half < 2; ++half) {
-        float a[2][8], b[2][8];
+        float a[NT][8], b[2][8];
 #pragma unroll
         for (int s = 0; s < 8; ++s) {
           const int row = 16 * half + chunk_k<PREC>(s, lk);
           if constexpr (!MPRE) {
-            a[0][s] = rt[row * 64 + li];
-            a[1][s] = rt[row * 64 + 32 + li];
+#pragma unroll
+            for (int t = 0; t < NT; ++t) a[t][s] = rt[row * W + 32 * t + li];
           }
           b[0][s] = jt[row * kPitch + 64 * wave + li];
           b[1][s] = jt[row * kPitch + 64 * wave + 32 + li];
@@ -856,7 +878,7 @@ __global__ __launch_bounds__(kBlock) void k_gemm_jtr(const float* __restrict__ J
     }
     flush(acc, tot);
 #pragma unroll
-    for (int ta = 0; ta < 2; ++ta)
+    for (int ta = 0; ta < NT; ++ta)
 #pragma unroll
       for (int tb = 0; tb < 2; ++tb) {
         const long c = cbase + 64 * wave + 32 * tb + li;
@@ -1377,7 +1399,7 @@ hipError_t run_jm(jgm_context* ctx, int gemm_precision, const float* Xt, int P, 
   const long R = (long)ctx->storedJ_rows;
   const long ld = (long)ctx->storedJ_ld;
   hipStream_t st = ctx->stream;
-  const int rhs_tiles = P / 64;
+  const int rhs_tiles = (P + 63) / 64;
   const int row_tiles = (int)((ld + 255) / 256);
   const bool streamed = storedj_streamed(ctx);
   hipError_t e;
@@ -1428,7 +1450,14 @@ hipError_t run_jm(jgm_context* ctx, int gemm_precision, const float* Xt, int P, 
                      (const bf16x8*)nullptr, (const bf16x8*)nullptr, P, per, row_tiles,      \
                      (int)nsplit, ctx->partial.as<float>())
       switch (gemm_precision) {
-        case JGM_GEMM_FP32: JGM_JM(JGM_GEMM_FP32); break;
+        case JGM_GEMM_FP32:
+          if (P == 32)
+            hipLaunchKernelGGL((k_gemm_jm<JGM_GEMM_FP32, false, 1>), grid, dim3(kBlock), 0, st, J,
+                               ld, R, ncols, Mt, (const bf16x8*)nullptr, (const bf16x8*)nullptr,
+                               P, per, row_tiles, (int)nsplit, ctx->partial.as<float>());
+          else
+            JGM_JM(JGM_GEMM_FP32);
+          break;
         case JGM_GEMM_BF16:
           if (packed)
             hipLaunchKernelGGL(k_gemm_jm_bf16p, grid, dim3(kBlock), 0, st,
@@ -1497,18 +1526,23 @@ hipError_t run_jtr(jgm_context* ctx, int gemm_precision, const float* Xt, int P,
     const long nblk = ncols / kColPad;
     const long nvalid = std::max<long>(0, std::min(ncols, N - c0));
     if (nvalid == 0) return hipSuccess;
-    dim3 grid((unsigned)std::min<long>(nblk, 65535), (unsigned)(P / 64));
+    dim3 grid((unsigned)std::min<long>(nblk, 65535), (unsigned)((P + 63) / 64));
     ProfScope ps(ctx, gemm_precision == JGM_GEMM_FP32   ? "storedj_jtr_fp32"
                       : gemm_precision == JGM_GEMM_BF16 ? "storedj_jtr_bf16"
                                                         : "storedj_jtr_bf16_refined");
-#define JGM_JTR(PR, PRE)                                                                     \
-  hipLaunchKernelGGL((k_gemm_jtr<PR, PRE>), grid, dim3(kBlock), 0, st, J, ld, nvalid, nblk, Xt, \
+#define JGM_JTR(PR, PRE, NT)                                                                 \
+  hipLaunchKernelGGL((k_gemm_jtr<PR, PRE, NT>), grid, dim3(kBlock), 0, st, J, ld, nvalid, nblk, Xt, \
                      ctx->storedJ_rhs16.as<const bf16x8>(),                                 \
                      ctx->storedJ_rhs16lo.as<const bf16x8>(), P, out + c0, N, nrhs)
     switch (gemm_precision) {
-      case JGM_GEMM_FP32: JGM_JTR(JGM_GEMM_FP32, false); break;
-      case JGM_GEMM_BF16: JGM_JTR(JGM_GEMM_BF16, false); break;
-      default: JGM_JTR(JGM_GEMM_BF16_REFINED, true); break;
+      case JGM_GEMM_FP32:
+        if (P == 32)
+          JGM_JTR(JGM_GEMM_FP32, false, 1);
+        else
+          JGM_JTR(JGM_GEMM_FP32, false, 2);
+        break;
+      case JGM_GEMM_BF16: JGM_JTR(JGM_GEMM_BF16, false, 2); break;
+      default: JGM_JTR(JGM_GEMM_BF16_REFINED, true, 2); break;
     }
 #undef JGM_JTR
     return hipGetLastError();
@@ -1529,66 +1563,74 @@ __device__ __forceinline__ f64x4 mfma_f64(double a, double b, f64x4 c) {
   return __builtin_amdgcn_mfma_f64_16x16x4f64(a, b, c, 0, 0, 0);
 }
 
+// NU: tiles of 16 right-hand sides (1 for at most 16 of them, else 4)
+template <int NU>
 struct Frag64 {
-  double a[4][4], b[4][4];  // [k-step][tile]
+  double a[4][4], b[4][NU];  // [k-step][tile]
 };
 // register stages of k_gemm_jm_f64: 3 (206 VGPRs with the 128 accumulator AGPRs still 1
-// wave per SIMD) reads FP64 J 13 % faster than 2; 4 would spill
-constexpr int kJm64Stages = 3;
+// wave per SIMD) reads FP64 J 13 % faster than 2; 4 would spill.  One right-hand-side tile
+// leaves registers for 5.
+template <int NU>
+constexpr int kJm64Stages = NU == 1 ? 5 : 3;
 
-__device__ __forceinline__ void mma64(const Frag64& f, f64x4 (&acc)[4][4]) {
+template <int NU>
+__device__ __forceinline__ void mma64(const Frag64<NU>& f, f64x4 (&acc)[4][NU]) {
 #pragma unroll
   for (int s = 0; s < 4; ++s)
 #pragma unroll
     for (int t = 0; t < 4; ++t)
 #pragma unroll
-      for (int u = 0; u < 4; ++u) acc[t][u] = mfma_f64(f.a[s][t], f.b[s][u], acc[t][u]);
+      for (int u = 0; u < NU; ++u) acc[t][u] = mfma_f64(f.a[s][t], f.b[s][u], acc[t][u]);
 }
 
 // Y partials Yp[split][row][P] (FP64) of J M; grid and split layout as k_gemm_jm.
+template <int NU>
 __global__ __launch_bounds__(kBlock) void k_gemm_jm_f64(const double* __restrict__ J, long ld,
                                                         long R, long colpad,
                                                         const double* __restrict__ Mt, int P,
                                                         long per, int row_tiles, int nsplit,
                                                         double* __restrict__ Yp) {
   const int w = blockIdx.x;
+  constexpr int NS = kJm64Stages<NU>;
   int split, rt;
   xcd_item(w, nsplit * row_tiles, row_tiles, split, rt);
   const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
   const int li = lane & 15, g = lane >> 4;
   const long row0 = (long)rt * 256 + wave * 64;
   if (row0 >= ld) return;  // whole wave outside the padded rows; no barriers follow
-  const int b0 = blockIdx.y * 64;
+  const int b0 = blockIdx.y * 16 * NU;
   const long c0 = (long)split * per;
   const long cend = c0 + per < colpad ? c0 + per : colpad;
   const int nchunk = cend > c0 ? (int)((cend - c0) / kChunk) : 0;
-  const double* Jw = J + row0 + li;
+  const double* Jw = J + row0 + 4 * li;
   const double* Mw = Mt + b0 + li;
-  f64x4 acc[4][4];
+  f64x4 acc[4][NU];
 #pragma unroll
   for (int t = 0; t < 4; ++t)
 #pragma unroll
-    for (int u = 0; u < 4; ++u) acc[t][u] = f64x4{0.0, 0.0, 0.0, 0.0};
-  // a ring of kJm64Stages chunks in registers, as in k_gemm_jm
-  Frag64 f[kJm64Stages];
-  auto load = [&](Frag64& h, int q) {
+    for (int u = 0; u < NU; ++u) acc[t][u] = f64x4{0.0, 0.0, 0.0, 0.0};
+  // a ring of NS chunks in registers, as in k_gemm_jm
+  Frag64<NU> f[NS];
+  auto load = [&](Frag64<NU>& h, int q) {
     const long cb = c0 + (long)(q < nchunk ? q : nchunk - 1) * kChunk;  // past the end: unused
 #pragma unroll
     for (int st = 0; st < 4; ++st) {
       const long cell = cb + 4 * g + st;
+      const f64x4 v = __builtin_nontemporal_load((const f64x4*)(Jw + cell * ld));
 #pragma unroll
-      for (int t = 0; t < 4; ++t) h.a[st][t] = __builtin_nontemporal_load(Jw + cell * ld + 16 * t);
+      for (int t = 0; t < 4; ++t) h.a[st][t] = v[t];
 #pragma unroll
-      for (int u = 0; u < 4; ++u) h.b[st][u] = Mw[cell * P + 16 * u];
+      for (int u = 0; u < NU; ++u) h.b[st][u] = Mw[cell * P + 16 * u];
     }
   };
   if (nchunk > 0) {
 #pragma unroll
-    for (int d = 0; d < kJm64Stages - 1; ++d) load(f[d], d);
-    for (int q = 0; q < nchunk; q += kJm64Stages) {
+    for (int d = 0; d < NS - 1; ++d) load(f[d], d);
+    for (int q = 0; q < nchunk; q += NS) {
 #pragma unroll
-      for (int d = 0; d < kJm64Stages; ++d) {
-        load(f[(d + kJm64Stages - 1) % kJm64Stages], q + d + kJm64Stages - 1);
+      for (int d = 0; d < NS; ++d) {
+        load(f[(d + NS - 1) % NS], q + d + NS - 1);
         __builtin_amdgcn_sched_barrier(0);
         if (q + d < nchunk) mma64(f[d], acc);
         __builtin_amdgcn_sched_barrier(0);
@@ -1600,10 +1642,10 @@ __global__ __launch_bounds__(kBlock) void k_gemm_jm_f64(const double* __restrict
   for (int t = 0; t < 4; ++t)
 #pragma unroll
     for (int r = 0; r < 4; ++r) {
-      const long row = row0 + 16 * t + g + 4 * r;
+      const long row = row0 + 4 * (g + 4 * r) + t;  // row i of tile t is the wave's row 4 i + t
       if (row < R) {
 #pragma unroll
-        for (int u = 0; u < 4; ++u) out[row * P + b0 + 16 * u + li] = acc[t][u][r];
+        for (int u = 0; u < NU; ++u) out[row * P + b0 + 16 * u + li] = acc[t][u][r];
       }
     }
 }
@@ -1625,6 +1667,7 @@ __global__ __launch_bounds__(kBlock) void k_gemm_jm_reduce_f64(const double* __r
 // A = J^T (i = cell, k = row): a lane's four rows of a chunk are one 32-byte load from its
 // cell's column; B = Rt (k = row, j = right-hand side).  The next chunk's loads are in
 // flight while the current one is multiplied.
+template <int NU>
 __global__ __launch_bounds__(kBlock) void k_gemm_jtr_f64(const double* __restrict__ J, long ld,
                                                          long N, long nblk,
                                                          const double* __restrict__ Rt, int P,
@@ -1632,41 +1675,44 @@ __global__ __launch_bounds__(kBlock) void k_gemm_jtr_f64(const double* __restric
                                                          int nrhs) {
   const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
   const int li = lane & 15, g = lane >> 4;
-  const int b0 = blockIdx.y * 64;
-  const long nchunk = ld / kChunk;  // even: ld is a multiple of 64
+  const int b0 = blockIdx.y * 16 * NU;
+  const long nchunk = ld / kChunk;
   for (long blk = blockIdx.x; blk < nblk; blk += gridDim.x) {
     const long cbase = blk * kColPad + 64 * wave;
     const double* Jw = J + (cbase + li) * ld + 4 * g;
     const double* Rw = Rt + (long)(4 * g) * P + b0 + li;
-    f64x4 acc[4][4];
+    f64x4 acc[4][NU];
 #pragma unroll
     for (int t = 0; t < 4; ++t)
 #pragma unroll
-      for (int u = 0; u < 4; ++u) acc[t][u] = f64x4{0.0, 0.0, 0.0, 0.0};
-    Frag64 x, y;
-    auto load = [&](Frag64& f, long rb) {
+      for (int u = 0; u < NU; ++u) acc[t][u] = f64x4{0.0, 0.0, 0.0, 0.0};
+    // a ring of register stages: two, or four for one right-hand-side tile (ld is a multiple
+    // of 64, so nchunk is one of 4)
+    constexpr int NS = NU == 1 ? 4 : 2;
+    Frag64<NU> f[NS];
+    auto load = [&](Frag64<NU>& h, long rb) {
 #pragma unroll
       for (int t = 0; t < 4; ++t) {
         const f64x4 v = __builtin_nontemporal_load((const f64x4*)(Jw + (long)16 * t * ld + rb));
 #pragma unroll
-        for (int st = 0; st < 4; ++st) f.a[st][t] = v[st];
+        for (int st = 0; st < 4; ++st) h.a[st][t] = v[st];
       }
 #pragma unroll
       for (int st = 0; st < 4; ++st)
 #pragma unroll
-        for (int u = 0; u < 4; ++u) f.b[st][u] = Rw[(rb + st) * P + 16 * u];
+        for (int u = 0; u < NU; ++u) h.b[st][u] = Rw[(rb + st) * P + 16 * u];
     };
-    load(x, 0);
-    for (long q = 0; q < nchunk; q += 2) {
-      load(y, (q + 1) * kChunk);
-      __builtin_amdgcn_sched_barrier(0);
-      mma64(x, acc);
-      __builtin_amdgcn_sched_barrier(0);
-      const long qn = q + 2 < nchunk ? q + 2 : nchunk - 1;  // the last reload is unused
-      load(x, qn * kChunk);
-      __builtin_amdgcn_sched_barrier(0);
-      mma64(y, acc);
-      __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int d = 0; d < NS - 1; ++d) load(f[d], d * kChunk);
+    for (long q = 0; q < nchunk; q += NS) {
+#pragma unroll
+      for (int d = 0; d < NS; ++d) {
+        const long qn = q + d + NS - 1 < nchunk ? q + d + NS - 1 : nchunk - 1;  // past the end: unused
+        load(f[(d + NS - 1) % NS], qn * kChunk);
+        __builtin_amdgcn_sched_barrier(0);
+        mma64(f[d], acc);
+        __builtin_amdgcn_sched_barrier(0);
+      }
     }
 #pragma unroll
     for (int t = 0; t < 4; ++t)
@@ -1675,7 +1721,7 @@ __global__ __launch_bounds__(kBlock) void k_gemm_jtr_f64(const double* __restric
         const long c = cbase + 16 * t + g + 4 * r;
         if (c < N) {
 #pragma unroll
-          for (int u = 0; u < 4; ++u) {
+          for (int u = 0; u < NU; ++u) {
             const int b = b0 + 16 * u + li;
             if (b < nrhs) G[c + (long)b * ldg] = acc[t][u][r];
           }
@@ -1688,7 +1734,7 @@ __global__ __launch_bounds__(kBlock) void k_gemm_jtr_f64(const double* __restric
 hipError_t run_jm_f64(jgm_context* ctx, const double* Xt, int P, int nrhs, double* out) {
   const long R = (long)ctx->storedJ_rows, ld = (long)ctx->storedJ_ld;
   const long colpad = (long)ctx->storedJ_colpad;
-  const int rhs_tiles = P / 64;
+  const int rhs_tiles = (P + 63) / 64;
   const int row_tiles = (int)((ld + 255) / 256);
   // one pass of workgroups over the CUs (one per CU at 1 wave per SIMD): on 7168 x 65536,
   // 9 splits run 1.02 ms against 1.12 ms for 16 (448 workgroups: a second pass three
@@ -1700,9 +1746,11 @@ hipError_t run_jm_f64(jgm_context* ctx, const double* Xt, int P, int nrhs, doubl
   if (e != hipSuccess) return e;
   {
     ProfScope ps(ctx, "storedj_jm_fp64");
-    hipLaunchKernelGGL(k_gemm_jm_f64, dim3((unsigned)(nsplit * row_tiles), (unsigned)rhs_tiles),
-                       dim3(kBlock), 0, ctx->stream, ctx->storedJ.as<const double>(), ld, R,
-                       colpad, Xt, P, per, row_tiles, (int)nsplit, ctx->partial.as<double>());
+    const dim3 grid((unsigned)(nsplit * row_tiles), (unsigned)rhs_tiles);
+    const auto kernel = P == 16 ? k_gemm_jm_f64<1> : k_gemm_jm_f64<4>;
+    hipLaunchKernelGGL(kernel, grid, dim3(kBlock), 0, ctx->stream, ctx->storedJ.as<const double>(),
+                       ld, R, colpad, Xt, P, per, row_tiles, (int)nsplit,
+                       ctx->partial.as<double>());
   }
   hipLaunchKernelGGL(k_gemm_jm_reduce_f64, dim3(blocks_for(R * (long)nrhs)), dim3(kBlock), 0,
                      ctx->stream, ctx->partial.as<const double>(), (int)nsplit, R, P, nrhs, out);
@@ -1714,9 +1762,10 @@ hipError_t run_jtr_f64(jgm_context* ctx, const double* Xt, int P, int nrhs, doub
   const long N = (long)ctx->storedJ_cols, ld = (long)ctx->storedJ_ld;
   const long nblk = (long)ctx->storedJ_colpad / kColPad;
   ProfScope ps(ctx, "storedj_jtr_fp64");
-  hipLaunchKernelGGL(k_gemm_jtr_f64, dim3((unsigned)std::min<long>(nblk, 65535), (unsigned)(P / 64)),
-                     dim3(kBlock), 0, ctx->stream, ctx->storedJ.as<const double>(), ld, N, nblk,
-                     Xt, P, out, N, nrhs);
+  const dim3 grid((unsigned)std::min<long>(nblk, 65535), (unsigned)((P + 63) / 64));
+  const auto kernel = P == 16 ? k_gemm_jtr_f64<1> : k_gemm_jtr_f64<4>;
+  hipLaunchKernelGGL(kernel, grid, dim3(kBlock), 0, ctx->stream, ctx->storedJ.as<const double>(),
+                     ld, N, nblk, Xt, P, out, N, nrhs);
   return hipGetLastError();
 }
 
@@ -1726,7 +1775,7 @@ hipError_t launch_storedj_apply_f64(jgm_context* ctx, int transpose, const doubl
                                     size_t nrhs, double* out) {
   const long R = (long)ctx->storedJ_rows, N = (long)ctx->storedJ_cols;
   const long ld = (long)ctx->storedJ_ld, colpad = (long)ctx->storedJ_colpad;
-  const int P = (int)round_up((long)nrhs, 64);
+  const int P = rhs_pad(JGM_GEMM_FP64, true, (long)nrhs);
   const long K = transpose ? R : N, Kpad = transpose ? ld : colpad;
   hipError_t e = ctx->coef32.ensure(sizeof(double) * (size_t)Kpad * P);
   if (e != hipSuccess) return e;
@@ -1741,7 +1790,7 @@ hipError_t launch_storedj_apply(jgm_context* ctx, int gemm_precision, int transp
                                 const float* in, size_t nrhs, float* out) {
   const long R = (long)ctx->storedJ_rows, N = (long)ctx->storedJ_cols;
   const long ld = (long)ctx->storedJ_ld, colpad = (long)ctx->storedJ_colpad;
-  const int P = (int)round_up((long)nrhs, 64);
+  const int P = rhs_pad(gemm_precision, false, (long)nrhs);
   const long K = transpose ? R : N, Kpad = transpose ? ld : colpad;
   hipError_t e = ctx->coef32.ensure(sizeof(float) * (size_t)Kpad * P);
   if (e != hipSuccess) return e;
@@ -1787,10 +1836,11 @@ hipError_t forward_batch_impl(jgm_context* ctx, int gemm_precision, size_t nmode
   const int kind = ctx->storedJ_kind;
   const int S = (int)ctx->S;
   const int L = has_background(kind) ? (int)ctx->bgthick.size() : 0;
-  const int P = 64;
-  hipError_t e = ctx->coef32.ensure(sizeof(T) * (size_t)colpad * P);
+  constexpr size_t kGroup = 64;
+  const size_t nb_max = std::min<size_t>(nmodels, kGroup);
+  hipError_t e = ctx->coef32.ensure(
+      sizeof(T) * (size_t)colpad * rhs_pad(gemm_precision, sizeof(T) == 8, (long)nb_max));
   if (e != hipSuccess) return e;
-  const size_t nb_max = std::min<size_t>(nmodels, (size_t)P);
   if ((e = ctx->storedJ_vec.ensure(sizeof(T) * (size_t)std::max(R * (long)nb_max, N))) !=
       hipSuccess)
     return e;
@@ -1798,8 +1848,9 @@ hipError_t forward_batch_impl(jgm_context* ctx, int gemm_precision, size_t nmode
   const double tf_bx = std::cos(ctx->tf_inc) * std::cos(ctx->tf_dec);
   const double tf_by = std::cos(ctx->tf_inc) * std::sin(ctx->tf_dec);
   const double tf_bz = std::sin(ctx->tf_inc);
-  for (size_t b0 = 0; b0 < nmodels; b0 += P) {
-    const int nb = (int)std::min<size_t>(nmodels - b0, (size_t)P);
+  for (size_t b0 = 0; b0 < nmodels; b0 += kGroup) {
+    const int nb = (int)std::min<size_t>(nmodels - b0, kGroup);
+    const int P = rhs_pad(gemm_precision, sizeof(T) == 8, nb);
     const double* m = models + b0 * model_ld;
     hipLaunchKernelGGL(k_vec_to_rhs<T>, dim3(blocks_for(colpad * P)), dim3(kBlock), 0,
                        ctx->stream, m, (long)model_ld, nb, N, colpad, P, Xt);
@@ -1823,16 +1874,18 @@ hipError_t gradient_batch_impl(jgm_context* ctx, int gemm_precision, size_t nset
   const long R = (long)ctx->storedJ_rows, N = (long)ctx->storedJ_cols;
   const long ld = (long)ctx->storedJ_ld;
   const int kind = ctx->storedJ_kind;
-  const int P = 64;
-  hipError_t e = ctx->coef32.ensure(sizeof(T) * (size_t)ld * P);
+  constexpr size_t kGroup = 64;
+  const size_t nb_max = std::min<size_t>(nsets, kGroup);
+  hipError_t e = ctx->coef32.ensure(
+      sizeof(T) * (size_t)ld * rhs_pad(gemm_precision, sizeof(T) == 8, (long)nb_max));
   if (e != hipSuccess) return e;
-  const size_t nb_max = std::min<size_t>(nsets, (size_t)P);
   if ((e = ctx->storedJ_vec.ensure(sizeof(T) * (size_t)std::max(R, N * (long)nb_max))) !=
       hipSuccess)
     return e;
   T* Xt = ctx->coef32.as<T>();
-  for (size_t b0 = 0; b0 < nsets; b0 += P) {
-    const int nb = (int)std::min<size_t>(nsets - b0, (size_t)P);
+  for (size_t b0 = 0; b0 < nsets; b0 += kGroup) {
+    const int nb = (int)std::min<size_t>(nsets - b0, kGroup);
+    const int P = rhs_pad(gemm_precision, sizeof(T) == 8, nb);
     const double* rm = raw_misfits + b0 * misfit_ld;
     hipLaunchKernelGGL(k_rm_to_compact<T>, dim3(blocks_for(ld * P)), dim3(kBlock), 0,
                        ctx->stream, rm, (long)misfit_ld, nb, (int)ctx->S, kind, ld, P, Xt);
