@@ -9,7 +9,15 @@ q is the degree-7 polynomial that minimises its own largest relative error (q(x)
 
 Both by Remez exchange at 60 significant digits, rounded to doubles.  Run
 `python jif3d_amd/csrc/corner_poly.py` to print them and the errors they leave.
+
+log by table (LogTable): 256 intervals of the mantissa m in [1/2, 1), each with a reciprocal
+inv (a multiple of 2^-9 near 1/m) and -log(inv) = hi + lo, hi a multiple of 2^-42 so that
+e ln2_hi + hi is exact.  The first and last interval take inv = 2 and 1, so that f = m inv - 1
+is exact and the logarithm keeps its relative accuracy next to 1 on both sides.
+`python jif3d_amd/csrc/corner_poly.py --log-table` prints log_table.hpp.
 """
+import sys
+
 import mpmath as mp
 
 mp.mp.dps = 60
@@ -68,7 +76,38 @@ def log_q(x):
     return (mp.atanh(r) / r - 1) / x
 
 
+LN2_HI, LN2_LO = 6.93147180369123816490e-01, 1.90821492927058770002e-10  # prism_device.hpp
+
+
+def log_table():
+    """[(inv, hi, lo)] of the 256 mantissa intervals [1/2 + j 2^-9, 1/2 + (j + 1) 2^-9)."""
+    rows = []
+    for j in range(256):
+        if j == 0:  # -log 2 in the same two parts that e ln 2 is added in: cancels exactly
+            rows.append((2.0, -LN2_HI, -LN2_LO))
+            continue
+        mid = mp.mpf(1) / 2 + (mp.mpf(j) + mp.mpf(1) / 2) / 512
+        inv = mp.mpf(1) if j == 255 else mp.nint(512 / mid) / 512
+        value = -mp.log(inv)
+        hi = mp.nint(value * 2 ** 42) / mp.mpf(2) ** 42
+        rows.append((float(inv), float(hi), float(value - hi)))
+    return rows
+
+
+def print_log_table():
+    print("// Generated by `python jif3d_amd/csrc/corner_poly.py --log-table`: inv, hi, lo of the 256")
+    print("// mantissa intervals of LogTable (prism_device.hpp).")
+    print("#pragma once\n\n#include <hip/hip_runtime.h>\n\nnamespace jgm {\n")
+    print("static __device__ const double kLogTable[256][3] = {")
+    for inv, hi, lo in log_table():
+        print(f"    {{{inv!r}, {hi!r}, {lo!r}}},")
+    print("};\n\n}  // namespace jgm")
+
+
 def main():
+    if "--log-table" in sys.argv[1:]:
+        print_log_table()
+        return
     c, e = remez(atan_g, atan_weight, mp.tan(mp.pi / 8) ** 2, ATAN_DEG)
     print(f"# atan: max relative error of atan from g (exact arithmetic) {mp.nstr(e, 3)}")
     for k, ck in enumerate(c):

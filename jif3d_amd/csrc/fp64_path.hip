@@ -71,6 +71,8 @@ __global__ __launch_bounds__(kBlock) void k_forward_corners(
     const double* __restrict__ Zc, int ncy, int ncz, const double* __restrict__ w, long ncols,
     long cols_per_chunk, double* __restrict__ partial) {
   constexpr int NC = Ncomp<MASK>::value;
+  __shared__ typename CornerLog<MASK>::type tab;
+  const auto lg = tab.fill();
   const int s = blockIdx.x * blockDim.x + threadIdx.x;
   const int sl = s < S ? s : S - 1;
   const double px = sx[sl], py = sy[sl], pz = sz[sl];
@@ -90,7 +92,7 @@ __global__ __launch_bounds__(kBlock) void k_forward_corners(
     for (int K = 0; K < ncz; ++K) {
       const double z = pz - Zc[K];
       double t[NC];
-      corner_terms_f64<MASK>(x, y, z, t);
+      corner_terms_f64<MASK>(x, y, z, t, lg);
 #pragma unroll
       for (int b = 0; b < NB; ++b) {
         const double wk = wc[K * NB + b];
@@ -239,6 +241,8 @@ __global__ __launch_bounds__(kBlock) void k_adjoint_corners(
     const double* __restrict__ Xc, const double* __restrict__ Yc,
     const double* __restrict__ Zc, int ncy, int ncz, long ncorner, double* __restrict__ hpart) {
   constexpr int NC = Ncomp<MASK>::value;
+  __shared__ typename CornerLog<MASK>::type tab;
+  const auto lg = tab.fill();
   const long q = (long)blockIdx.x * blockDim.x + threadIdx.x;
   const long ql = q < ncorner ? q : ncorner - 1;
   const int K = (int)(ql % ncz);
@@ -254,7 +258,7 @@ __global__ __launch_bounds__(kBlock) void k_adjoint_corners(
   for (int s = s0; s < s1; ++s) {
     const double x = sx[s] - cx, y = sy[s] - cy, z = sz[s] - cz;
     double tv[NC];
-    corner_terms_f64<MASK>(x, y, z, tv);
+    corner_terms_f64<MASK>(x, y, z, tv, lg);
     const double* cs = coef + (long)s * NB * NC;
 #pragma unroll
     for (int b = 0; b < NB; ++b)
@@ -591,7 +595,7 @@ hipError_t adjoint_impl(jgm_context* ctx, int kind, int nb, const double* rm, si
 // Magnetic vertical gradient (OMPMagneticGradImp.cpp:13-106) and magnetization
 // (OMPMagnetizationImp.cpp:25-117).  The vertical gradient is the difference of the
 // susceptibility Bz at the site and 1 m below it, so both positions run through the
-// tensor corner kernels as 2S virtual sites.  The magnetization model has three values
+// corner kernels of the tensor's z column (kMaskZder) as 2S virtual sites.  The magnetization model has three values
 // per cell, B = 1e9 mu0/(4 pi G) T M, evaluated corner-first with three corner weight
 // sets in one pass.
 // ---------------------------------------------------------------------------
@@ -609,7 +613,7 @@ __global__ __launch_bounds__(kBlock) void k_pair_sites(const double* __restrict_
   vs[4 * S + v] = sz[s] + (v < S ? 0.0 : dz);
 }
 
-// Bz projection of the tensor kernel's components (xx, yy, zz, xy, xz, yz):
+// Bz projection of the z column's components (zz, xz, yz):
 // (T b)_z = Uxz bx + Uyz by + Uzz bz, times F mu0/(4 pi) / G = F 1e-7 / G.
 // dst[i] += src[i]
 __global__ __launch_bounds__(kBlock) void k_add_f64(double* __restrict__ dst,
@@ -632,9 +636,9 @@ __global__ __launch_bounds__(kBlock) void k_maggrad_finish(const double* __restr
     const int v = s + h * S;
     double zz = 0.0, xz = 0.0, yz = 0.0;
     for (int c = 0; c < nchunks; ++c) {
-      zz += partial[((long)c * 6 + 2) * S2 + v];
-      xz += partial[((long)c * 6 + 4) * S2 + v];
-      yz += partial[((long)c * 6 + 5) * S2 + v];
+      zz += partial[((long)c * 3 + 0) * S2 + v];
+      xz += partial[((long)c * 3 + 1) * S2 + v];
+      yz += partial[((long)c * 3 + 2) * S2 + v];
     }
     // tensor signs: diagonal +G, off-diagonal -G (BasicGravElements.cpp:151, :201)
     bz[h] = (-kGravConst * xz * fd.bx - kGravConst * yz * fd.by + kGravConst * zz * fd.bz) *
@@ -657,13 +661,10 @@ __global__ __launch_bounds__(kBlock) void k_maggrad_coef(const double* __restric
   const int s = v < S ? v : v - S;
   const double rs = rm[idx ? idx[s] : s];
   const double r = (v < S ? rs : -rs) * fs * (1e-7 / kGravConst);
-  double* c = coef + (long)v * 6;  // xx, yy, zz, xy, xz, yz with their sign * G
-  c[0] = 0.0;
-  c[1] = 0.0;
-  c[2] = r * fd.bz * kGravConst;
-  c[3] = 0.0;
-  c[4] = -r * fd.bx * kGravConst;
-  c[5] = -r * fd.by * kGravConst;
+  double* c = coef + (long)v * 3;  // zz, xz, yz with their sign * G
+  c[0] = r * fd.bz * kGravConst;
+  c[1] = -r * fd.bx * kGravConst;
+  c[2] = -r * fd.by * kGravConst;
 }
 
 // B_i = sum_j T_ij w_j over corners, T_ij = sign_ij F_ij (G and the unit factor
@@ -673,6 +674,8 @@ __global__ __launch_bounds__(kBlock) void k_forward_corners_mag3(
     int S, const double* __restrict__ Xc, const double* __restrict__ Yc,
     const double* __restrict__ Zc, int ncy, int ncz, const double* __restrict__ w, long nq,
     long ncols, long cols_per_chunk, double* __restrict__ partial) {
+  __shared__ LogTableShared tab;
+  const auto lg = tab.fill();
   const int s = blockIdx.x * blockDim.x + threadIdx.x;
   const int sl = s < S ? s : S - 1;
   const double px = sx[sl], py = sy[sl], pz = sz[sl];
@@ -689,7 +692,7 @@ __global__ __launch_bounds__(kBlock) void k_forward_corners_mag3(
       const double z = pz - Zc[K];
       const double wx = wc[K], wy = wc[nq + K], wz = wc[2 * nq + K];
       double t[6];  // xx, yy, zz, xy, xz, yz
-      corner_terms_f64<kMaskTensor>(x, y, z, t);
+      corner_terms_f64<kMaskTensor>(x, y, z, t, lg);
       bx += t[0] * wx - t[3] * wy - t[4] * wz;
       by += -t[3] * wx + t[1] * wy - t[5] * wz;
       bz += -t[4] * wx - t[5] * wy + t[2] * wz;
@@ -720,6 +723,8 @@ __global__ __launch_bounds__(kBlock) void k_adjoint_corners_mag3(
     const double* __restrict__ coef, int S, int sites_per_chunk,
     const double* __restrict__ Xc, const double* __restrict__ Yc,
     const double* __restrict__ Zc, int ncy, int ncz, long ncorner, double* __restrict__ hpart) {
+  __shared__ LogTableShared tab;
+  const auto lg = tab.fill();
   const long q = (long)blockIdx.x * blockDim.x + threadIdx.x;
   const long ql = q < ncorner ? q : ncorner - 1;
   const int K = (int)(ql % ncz);
@@ -732,7 +737,7 @@ __global__ __launch_bounds__(kBlock) void k_adjoint_corners_mag3(
   double hx = 0.0, hy = 0.0, hz = 0.0;
   for (int s = s0; s < s1; ++s) {
     double tv[6];
-    corner_terms_f64<kMaskTensor>(sx[s] - cx, sy[s] - cy, sz[s] - cz, tv);
+    corner_terms_f64<kMaskTensor>(sx[s] - cx, sy[s] - cy, sz[s] - cz, tv, lg);
     const double* c = coef + (long)s * 3;
     hx += c[0] * tv[0] - c[1] * tv[3] - c[2] * tv[4];
     hy += -c[0] * tv[3] + c[1] * tv[1] - c[2] * tv[5];
@@ -776,7 +781,7 @@ double magnetization_scale() {
 }
 
 // Vertical gradient at S listed sites (sx, sy, sz), written to rows idx[s] of out and
-// raw_out (rows s without idx): the tensor corner sums at the site and 1 m below.
+// raw_out (rows s without idx): the z column's corner sums at the site and 1 m below.
 hipError_t maggrad_forward_at(jgm_context* ctx, const double* model, int S, const double* sx,
                               const double* sy, const double* sz, const int* idx, double* out,
                               double* raw_out) {
@@ -793,21 +798,21 @@ hipError_t maggrad_forward_at(jgm_context* ctx, const double* model, int S, cons
   if (N > 0) {
     site_chunks(S2, ncols, &nchunks, &per);
     if ((e = ctx->weights.ensure(sizeof(double) * (size_t)ncols * ncz)) != hipSuccess) return e;
-    if ((e = ctx->partial.ensure(sizeof(double) * (size_t)nchunks * 6 * S2)) != hipSuccess)
+    if ((e = ctx->partial.ensure(sizeof(double) * (size_t)nchunks * 3 * S2)) != hipSuccess)
       return e;
     hipLaunchKernelGGL(k_corner_weights, dim3(blocks_for(ncols * ncz)), dim3(kBlock), 0, st,
                        model, 0L, 1, (int)ctx->nx, (int)ctx->ny, (int)ctx->nz,
                        ctx->weights.as<double>());
     const double* vs = ctx->vsites.as<const double>();
     ProfScope ps(ctx, "forward_corners_fp64_maggrad");
-    hipLaunchKernelGGL((k_forward_corners<kMaskTensor, 1>), dim3((S2 + kBlock - 1) / kBlock, nchunks),
+    hipLaunchKernelGGL((k_forward_corners<kMaskZder, 1>), dim3((S2 + kBlock - 1) / kBlock, nchunks),
                        dim3(kBlock), 0, st, vs, vs + S2, vs + 2 * S2, S2, ctx->d_Xc.as<double>(),
                        ctx->d_Yc.as<double>(), ctx->d_Zc.as<double>(), ncy, ncz,
                        ctx->weights.as<const double>(), ncols, per, ctx->partial.as<double>());
   }
   if (nchunks > 0) {
-    if ((e = ctx->partsum.ensure(sizeof(double) * 6 * (size_t)S2)) != hipSuccess) return e;
-    if ((e = launch_reduce_chunks(ctx, ctx->partial.as<const double>(), (int)nchunks, 6L * S2,
+    if ((e = ctx->partsum.ensure(sizeof(double) * 3 * (size_t)S2)) != hipSuccess) return e;
+    if ((e = launch_reduce_chunks(ctx, ctx->partial.as<const double>(), (int)nchunks, 3L * S2,
                                   ctx->partsum.as<double>())) != hipSuccess)
       return e;
   }
@@ -842,7 +847,7 @@ hipError_t maggrad_adjoint_at(jgm_context* ctx, int S, const double* sx, const d
   }
   if (N == 0 || S == 0) return hipSuccess;
   if ((e = ctx->vsites.ensure(sizeof(double) * 6 * (size_t)S)) != hipSuccess) return e;
-  if ((e = ctx->coef.ensure(sizeof(double) * 6 * (size_t)S2)) != hipSuccess) return e;
+  if ((e = ctx->coef.ensure(sizeof(double) * 3 * (size_t)S2)) != hipSuccess) return e;
   hipLaunchKernelGGL(k_pair_sites, dim3(blocks_for(S2)), dim3(kBlock), 0, st, sx, sy, sz, S, 1.0,
                      ctx->vsites.as<double>());
   hipLaunchKernelGGL(k_maggrad_coef, dim3(blocks_for(S2)), dim3(kBlock), 0, st, rm, S,
@@ -853,7 +858,7 @@ hipError_t maggrad_adjoint_at(jgm_context* ctx, int S, const double* sx, const d
   const double* vs = ctx->vsites.as<const double>();
   {
     ProfScope ps(ctx, "adjoint_corners_fp64_maggrad");
-    hipLaunchKernelGGL((k_adjoint_corners<kMaskTensor, 1>), dim3(blocks_for(nq), nchunks),
+    hipLaunchKernelGGL((k_adjoint_corners<kMaskZder, 1>), dim3(blocks_for(nq), nchunks),
                        dim3(kBlock), 0, st, vs, vs + S2, vs + 2 * S2, ctx->coef.as<const double>(),
                        S2, per, ctx->d_Xc.as<double>(), ctx->d_Yc.as<double>(),
                        ctx->d_Zc.as<double>(), ncy, ncz, nq, ctx->hpart.as<double>());

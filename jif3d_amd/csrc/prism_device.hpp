@@ -19,6 +19,8 @@
 #include <cfloat>
 #include <cstdint>
 
+#include "log_table.hpp"
+
 namespace jgm {
 
 constexpr double kGravConst = 6.67428e-11;  // jif3D/Gravity/BasicGravElements.h:22
@@ -26,17 +28,21 @@ constexpr double kPi = 3.14159265358979323846;
 
 // Component masks of the corner function.  Component order inside kernels:
 // gz, Uxx, Uyy, Uzz, Uxy, Uxz, Uyz.  kZcol alone (never combined with the others) is the
-// tensor's z column, Uzz, Uxz, Uyz: the terms the vertical magnetic gradient needs.
-enum : int { kGz = 1, kDiag = 2, kOff = 4, kZcol = 8 };
+// tensor's z column, Uzz, Uxz, Uyz: the terms the vertical magnetic gradient needs.  kZder
+// alone is the same column with Uzz derived as the tensor mask derives it and log_pos_f64:
+// the FP64 vertical gradient, a small difference of two large sums, keeps the values that
+// the full tensor's evaluation gives, bit for bit.
+enum : int { kGz = 1, kDiag = 2, kOff = 4, kZcol = 8, kZder = 16 };
 constexpr int kMaskScalar = kGz;
 constexpr int kMaskTensor = kDiag | kOff;
 constexpr int kMaskAll = kGz | kDiag | kOff;
 constexpr int kMaskZcol = kZcol;
+constexpr int kMaskZder = kZder;
 
 template <int MASK>
 struct Ncomp {
   static constexpr int value = ((MASK & kGz) ? 1 : 0) + ((MASK & kDiag) ? 3 : 0) +
-                               ((MASK & kOff) ? 3 : 0) + ((MASK & kZcol) ? 3 : 0);
+                               ((MASK & kOff) ? 3 : 0) + ((MASK & (kZcol | kZder)) ? 3 : 0);
 };
 
 // Natural logarithm of a finite a >= DBL_EPSILON (the guarded log arguments of the
@@ -85,6 +91,80 @@ __device__ __forceinline__ double log_pos_f64(double a) {
   const double err = (hi - (sum - bb)) + (t - bb);
   const double lo = fma(t, q, fma(de, ln2_lo, 2.0 * flo)) + err;
   return sum + lo;
+}
+
+// The two logarithms a corner term can take: log_pos_f64, or the same range by table.
+struct LogPoly {
+  __device__ __forceinline__ double operator()(double a) const { return log_pos_f64(a); }
+};
+
+// Logarithm of a normal a > 0 from a 256-entry table in LDS (Tang's table-driven method, ACM
+// TOMS 16, 1990, with the reduced argument formed by one FMA): a = 2^e m, m in [1/2, 1), the
+// leading 8 fraction bits select inv ~ 1/m, f = m inv - 1 with |f| <= 2^-8, and
+// log a = (e ln2_hi + hi) + f + (f^2 q(f) + e ln2_lo + lo), the first sum exact (log_table.hpp),
+// q the Taylor series of (log(1 + f) - f)/f^2 to f^5 (what is left out is below 2^-66).  Against
+// an exact logarithm: at most 0.51 ulp over [1e-10, 1e5], also next to 1.  19 VALU
+// operations and two LDS reads against log_pos_f64's ~40 VALU operations: the FP64 corner
+// kernels are bound by the VALU and leave the LDS idle.
+struct LogTable {
+  const double2* ih;  // inv, hi
+  const double* lo;
+  __device__ __forceinline__ double operator()(double a) const {
+    const int j = (__double2hiint(a) >> 12) & 255;
+    const double m = __builtin_amdgcn_frexp_mant(a);
+    const double e = (double)__builtin_amdgcn_frexp_exp(a);
+    const double2 t = ih[j];
+    const double l = lo[j];
+    const double f = fma(m, t.x, -1.0);
+    const double k = fma(e, 6.93147180369123816490e-01, t.y);
+    const double hi = k + f;
+    const double err = f - (hi - k);
+    double q = 1.0 / 7.0;
+    q = fma(q, f, -1.0 / 6.0);
+    q = fma(q, f, 0.2);
+    q = fma(q, f, -0.25);
+    q = fma(q, f, 1.0 / 3.0);
+    q = fma(q, f, -0.5);
+    return hi + (fma(f * f, q, fma(e, 1.90821492927058770002e-10, l)) + err);
+  }
+};
+
+// LDS copy of the table, filled by the first 256 threads of a workgroup (ends in a barrier
+// that every thread reaches).
+struct LogTableShared {
+  double2 ih[256];
+  double lo[256];
+  __device__ __forceinline__ LogTable fill() {
+    for (int j = threadIdx.x; j < 256; j += blockDim.x) {
+      ih[j] = make_double2(kLogTable[j][0], kLogTable[j][1]);
+      lo[j] = kLogTable[j][2];
+    }
+    __syncthreads();
+    return {ih, lo};
+  }
+};
+
+struct LogPolyShared {
+  __device__ __forceinline__ LogPoly fill() { return {}; }
+};
+// what a corner kernel declares in LDS for its mask
+template <int MASK>
+struct CornerLog {
+  typedef LogTableShared type;
+};
+template <>
+struct CornerLog<kMaskZder> {
+  typedef LogPolyShared type;
+};
+
+// sqrt of x in [DBL_MIN, 1e300] (0 and infinity give NaN): the hardware reciprocal root, one
+// Newton step and one residual correction of the root, within 0.5 ulp + 2^-40 ulp; 9
+// operations against ~17 of the library's, which also scales subnormal arguments.
+__device__ __forceinline__ double sqrt_pos_f64(double x) {
+  double y = __builtin_amdgcn_rsq(x);
+  y = fma(0.5 * y, fma(-x * y, y, 1.0), y);
+  const double g = x * y;
+  return fma(0.5 * y, fma(-g, g, x), g);
 }
 
 // Arctangent of p / q in the quadrant of (q, p), atan2(p, q), for p and q of magnitudes in
@@ -163,10 +243,12 @@ __device__ __forceinline__ void diag_terms_f64(double x, double y, double z, dou
   *C = which == 2 ? t3 : t2;
 }
 
-template <int MASK>
-__device__ __forceinline__ void corner_terms_f64(double x, double y, double z, double* t) {
-  const double r = sqrt(x * x + y * y + z * z);
+template <int MASK, class Log = LogPoly>
+__device__ __forceinline__ void corner_terms_f64(double x, double y, double z, double* t,
+                                                 Log lg = {}) {
+  const double r2 = x * x + y * y + z * z;
   if constexpr (MASK == kMaskZcol) {
+    const double r = sqrt(r2);
     // Uzz = atan2(x y, z r), Uxz = log(max(y + r, eps)), Uyz = log(max(x + r, eps)); the
     // atan2 term evaluated directly (the tensor mask may derive it from its two others)
     t[0] = (fmin(fmin(fabs(x), fabs(y)), fabs(z)) >= 1e-140 && r >= DBL_EPSILON && r <= 1e140)
@@ -176,37 +258,66 @@ __device__ __forceinline__ void corner_terms_f64(double x, double y, double z, d
     t[2] = log_pos_f64(fmax(x + r, DBL_EPSILON));
     return;
   }
+  if constexpr (MASK == kMaskZder) {
+    const double r = sqrt(r2);
+    if (fmin(fmin(fabs(x), fabs(y)), fabs(z)) >= 1e-140 && r >= DBL_EPSILON && r <= 1e140) {
+      // the C of diag_terms_f64: derived where z is smallest in magnitude
+      const double ax = fabs(x), ay = fabs(y), az = fabs(z);
+      const bool derived = !(ax <= ay && ax <= az) && !(ay <= az);
+      t[0] = atan2_f64(derived ? y * z : x * y, derived ? x * r : z * r);
+      if (derived) {
+        const int neg = (x < 0.0) + (y < 0.0) + (z < 0.0);
+        const double K = neg <= 1 ? 0.5 * kPi : (neg == 2 ? -1.5 * kPi : 2.5 * kPi);
+        t[0] = (K - t[0]) - atan2_f64(x * z, y * r);
+      }
+    } else {
+      t[0] = atan2(x * y, z * r);
+    }
+    t[1] = lg(fmax(y + r, DBL_EPSILON));
+    t[2] = lg(fmax(x + r, DBL_EPSILON));
+    return;
+  }
+  if constexpr (MASK == kMaskScalar) {
+    // no zero coordinate, products of two offsets within atan2_f64's range, and arguments
+    // of the logarithms where the guarded ones equal them
+    const double r = sqrt_pos_f64(r2);
+    const double ay = y + r, ax = x + r;
+    if (fmin(fmin(fabs(x), fabs(y)), fabs(z)) >= 1e-140 && r >= DBL_EPSILON && r <= 1e140 &&
+        fmin(ax, ay) >= DBL_EPSILON) {
+      t[0] = fma(z, atan2_f64(z * r, x * y), fma(x, lg(ay), y * lg(ax)));
+      return;
+    }
+  }
   int k = 0;
   if constexpr ((MASK & kOff) != 0) {
-    const double lz = log_pos_f64(fmax(z + r, DBL_EPSILON));
-    const double ly = log_pos_f64(fmax(y + r, DBL_EPSILON));
-    const double lx = log_pos_f64(fmax(x + r, DBL_EPSILON));
-    if constexpr ((MASK & kDiag) != 0) {
-      double A, B, C, G;
-      // no zero coordinate, and every product of two offsets within atan2_f64's range
-      if (fmin(fmin(fabs(x), fabs(y)), fabs(z)) >= 1e-140 && r >= DBL_EPSILON && r <= 1e140) {
-        diag_terms_f64<MASK>(x, y, z, r, &A, &B, &C);
-        G = ((x * y < 0.0 && z < 0.0) ? -1.5 * kPi : 0.5 * kPi) - C;
-      } else {
-        A = atan2(y * z, x * r);
-        B = atan2(x * z, y * r);
-        C = atan2(x * y, z * r);
-        G = atan2(z * fmax(r, DBL_EPSILON), x * y);
-      }
-      if constexpr ((MASK & kGz) != 0) t[k++] = x * ly + y * lx + z * G;
-      t[k++] = A;
-      t[k++] = B;
-      t[k++] = C;
-    } else if constexpr ((MASK & kGz) != 0) {
-      const double rg = fmax(r, DBL_EPSILON);
-      double v = x * ly + y * lx;
-      v += z * atan2(z * rg, x * y);
-      t[k++] = v;
+    static_assert((MASK & kDiag) != 0, "the tensor's six components come together");
+    // no zero coordinate, and every product of two offsets within atan2_f64's range
+    double r = sqrt_pos_f64(r2);
+    const bool plain =
+        fmin(fmin(fabs(x), fabs(y)), fabs(z)) >= 1e-140 && r >= DBL_EPSILON && r <= 1e140;
+    if (!plain) r = sqrt(r2);
+    const double lz = lg(fmax(z + r, DBL_EPSILON));
+    const double ly = lg(fmax(y + r, DBL_EPSILON));
+    const double lx = lg(fmax(x + r, DBL_EPSILON));
+    double A, B, C, G;
+    if (plain) {
+      diag_terms_f64<MASK>(x, y, z, r, &A, &B, &C);
+      G = ((x * y < 0.0 && z < 0.0) ? -1.5 * kPi : 0.5 * kPi) - C;
+    } else {
+      A = atan2(y * z, x * r);
+      B = atan2(x * z, y * r);
+      C = atan2(x * y, z * r);
+      G = atan2(z * fmax(r, DBL_EPSILON), x * y);
     }
+    if constexpr ((MASK & kGz) != 0) t[k++] = x * ly + y * lx + z * G;
+    t[k++] = A;
+    t[k++] = B;
+    t[k++] = C;
     t[k++] = lz;
     t[k++] = ly;
     t[k++] = lx;
   } else {
+    const double r = sqrt(r2);
     if constexpr ((MASK & kGz) != 0) {
       const double rg = fmax(r, DBL_EPSILON);
       double v = x * log(y + rg) + y * log(x + rg);
@@ -236,9 +347,10 @@ __host__ __device__ inline void comp_scales(double* s) {
 // Full per-cell box term (8 corners) for the background boxes and the
 // per-cell sensitivity rows.  Returns sign-applied, G-scaled values in the
 // kernel's component order, like CalcGravBoxTerm / CalcTensorBoxTerm.
-template <int MASK>
+template <int MASK, class Log = LogPoly>
 __device__ inline void box_terms_f64(double mx, double my, double mz, double ux, double uy,
-                                     double uz, double sx, double sy, double sz, double* out) {
+                                     double uz, double sx, double sy, double sz, double* out,
+                                     Log lg = {}) {
   constexpr int NC = Ncomp<MASK>::value;
   double acc[NC];
 #pragma unroll
@@ -253,7 +365,7 @@ __device__ inline void box_terms_f64(double mx, double my, double mz, double ux,
   for (int n = 0; n < 8; ++n) {
     const int a = order[n][0], b = order[n][1], c = order[n][2];
     double t[NC];
-    corner_terms_f64<MASK>(xs[a], ys[b], zs[c], t);
+    corner_terms_f64<MASK>(xs[a], ys[b], zs[c], t, lg);
     if (n == 0) {
 #pragma unroll
       for (int m = 0; m < NC; ++m) acc[m] = -t[m];

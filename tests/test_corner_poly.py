@@ -93,3 +93,57 @@ def test_log_polynomial_on_the_reduced_range():
         q = q * x + np.longdouble(c)
     # q's relative error enters the logarithm scaled by x q <= 0.01: 5e-16 here is 0.05 ulp
     assert float(np.max(np.abs(q - exact) / exact)) <= 5e-16
+
+
+TABLE = os.path.join(os.path.dirname(HDR), "log_table.hpp")
+
+
+def log_table():
+    rows = re.findall(r"^    \{(\S+), (\S+), (\S+)\},$", open(TABLE).read(), re.M)
+    return np.array([[float(v) for v in r] for r in rows])
+
+
+def test_log_table_is_the_generators():
+    import importlib.util
+    path = os.path.join(os.path.dirname(HDR), "corner_poly.py")
+    spec = importlib.util.spec_from_file_location("corner_poly", path)
+    gen = importlib.util.module_from_spec(spec)
+    spec.loader.exec_module(gen)
+    assert np.array_equal(log_table(), np.array(gen.log_table()))
+
+
+def test_log_table_within_half_an_ulp():
+    """LogTable restated with its fused operations in extended precision (each is rounded
+    once to double), against the extended-precision logarithm: 0.52 ulp."""
+    t = log_table()
+    assert t.shape == (256, 3)
+    src = open(HDR).read()
+    body = src[src.index("struct LogTable {"):]
+    body = body[:body.index("\n};\n")]
+    q0 = eval(re.search(r"double q = (.+);", body).group(1))
+    rest = [eval(v) for v in re.findall(r"q = fma\(q, f, (.+)\);", body)]
+    ln2_hi, ln2_lo = 6.93147180369123816490e-01, 1.90821492927058770002e-10
+    assert body.count("6.93147180369123816490e-01") == 1
+    assert body.count("1.90821492927058770002e-10") == 1
+    ld = np.longdouble
+    rng = np.random.default_rng(0)
+    a = np.concatenate([np.exp(rng.uniform(-36, 12, 200000)), rng.uniform(0.99, 1.01, 100000),
+                        2.0 ** rng.integers(-52, 20, 1000).astype(float), 2.0 ** -52 * np.ones(1)])
+    m, e = np.frexp(a)
+    inv, hi_t, lo_t = t[((m - 0.5) * 512).astype(int)].T
+    f = (m.astype(ld) * inv - 1).astype(float)  # one rounding (63 bits hold the product)
+    k = (e.astype(ld) * ln2_hi + hi_t).astype(float)
+    assert np.array_equal(k.astype(ld), e.astype(ld) * ln2_hi + hi_t.astype(ld))  # exact
+    hi = k + f
+    err = f - (hi - k)
+    q = np.full_like(f, q0)
+    for c in rest:
+        q = (q.astype(ld) * f + c).astype(float)
+    w = (e.astype(ld) * ln2_lo + lo_t).astype(float)
+    w = ((f * f).astype(ld) * q + w).astype(float)
+    got = hi + (w + err)
+    ref = np.log(a.astype(ld))
+    one = a == 1.0
+    assert np.all(got[one] == 0.0)
+    ulp = np.spacing(np.abs(ref[~one].astype(float)))
+    assert float(np.max(np.abs(got[~one] - ref[~one]) / ulp)) <= 0.52
