@@ -71,8 +71,8 @@ __global__ __launch_bounds__(kBlock) void k_forward_corners(
     const double* __restrict__ Zc, int ncy, int ncz, const double* __restrict__ w, long ncols,
     long cols_per_chunk, double* __restrict__ partial) {
   constexpr int NC = Ncomp<MASK>::value;
-  __shared__ typename CornerLog<MASK>::type tab;
-  const auto lg = tab.fill();
+  __shared__ LogTableShared tab;
+  const LogTable lg = tab.fill();
   const int s = blockIdx.x * blockDim.x + threadIdx.x;
   const int sl = s < S ? s : S - 1;
   const double px = sx[sl], py = sy[sl], pz = sz[sl];
@@ -241,8 +241,8 @@ __global__ __launch_bounds__(kBlock) void k_adjoint_corners(
     const double* __restrict__ Xc, const double* __restrict__ Yc,
     const double* __restrict__ Zc, int ncy, int ncz, long ncorner, double* __restrict__ hpart) {
   constexpr int NC = Ncomp<MASK>::value;
-  __shared__ typename CornerLog<MASK>::type tab;
-  const auto lg = tab.fill();
+  __shared__ LogTableShared tab;
+  const LogTable lg = tab.fill();
   const long q = (long)blockIdx.x * blockDim.x + threadIdx.x;
   const long ql = q < ncorner ? q : ncorner - 1;
   const int K = (int)(ql % ncz);
@@ -675,7 +675,7 @@ __global__ __launch_bounds__(kBlock) void k_forward_corners_mag3(
     const double* __restrict__ Zc, int ncy, int ncz, const double* __restrict__ w, long nq,
     long ncols, long cols_per_chunk, double* __restrict__ partial) {
   __shared__ LogTableShared tab;
-  const auto lg = tab.fill();
+  const LogTable lg = tab.fill();
   const int s = blockIdx.x * blockDim.x + threadIdx.x;
   const int sl = s < S ? s : S - 1;
   const double px = sx[sl], py = sy[sl], pz = sz[sl];
@@ -724,7 +724,7 @@ __global__ __launch_bounds__(kBlock) void k_adjoint_corners_mag3(
     const double* __restrict__ Xc, const double* __restrict__ Yc,
     const double* __restrict__ Zc, int ncy, int ncz, long ncorner, double* __restrict__ hpart) {
   __shared__ LogTableShared tab;
-  const auto lg = tab.fill();
+  const LogTable lg = tab.fill();
   const long q = (long)blockIdx.x * blockDim.x + threadIdx.x;
   const long ql = q < ncorner ? q : ncorner - 1;
   const int K = (int)(ql % ncz);

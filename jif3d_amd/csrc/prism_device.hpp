@@ -29,9 +29,8 @@ constexpr double kPi = 3.14159265358979323846;
 // Component masks of the corner function.  Component order inside kernels:
 // gz, Uxx, Uyy, Uzz, Uxy, Uxz, Uyz.  kZcol alone (never combined with the others) is the
 // tensor's z column, Uzz, Uxz, Uyz: the terms the vertical magnetic gradient needs.  kZder
-// alone is the same column with Uzz derived as the tensor mask derives it and log_pos_f64:
-// the FP64 vertical gradient, a small difference of two large sums, keeps the values that
-// the full tensor's evaluation gives, bit for bit.
+// alone is the same column with Uzz derived as the tensor mask derives it: the FP64 vertical
+// gradient, a small difference of two large sums, keeps the full tensor's values.
 enum : int { kGz = 1, kDiag = 2, kOff = 4, kZcol = 8, kZder = 16 };
 constexpr int kMaskScalar = kGz;
 constexpr int kMaskTensor = kDiag | kOff;
@@ -144,19 +143,6 @@ struct LogTableShared {
   }
 };
 
-struct LogPolyShared {
-  __device__ __forceinline__ LogPoly fill() { return {}; }
-};
-// what a corner kernel declares in LDS for its mask
-template <int MASK>
-struct CornerLog {
-  typedef LogTableShared type;
-};
-template <>
-struct CornerLog<kMaskZder> {
-  typedef LogPolyShared type;
-};
-
 // sqrt of x in [DBL_MIN, 1e300] (0 and infinity give NaN): the hardware reciprocal root, one
 // Newton step and one residual correction of the root, within 0.5 ulp + 2^-40 ulp; 9
 // operations against ~17 of the library's, which also scales subnormal arguments.
@@ -259,7 +245,7 @@ __device__ __forceinline__ void corner_terms_f64(double x, double y, double z, d
     return;
   }
   if constexpr (MASK == kMaskZder) {
-    const double r = sqrt(r2);
+    double r = sqrt_pos_f64(r2);
     if (fmin(fmin(fabs(x), fabs(y)), fabs(z)) >= 1e-140 && r >= DBL_EPSILON && r <= 1e140) {
       // the C of diag_terms_f64: derived where z is smallest in magnitude
       const double ax = fabs(x), ay = fabs(y), az = fabs(z);
@@ -271,6 +257,7 @@ __device__ __forceinline__ void corner_terms_f64(double x, double y, double z, d
         t[0] = (K - t[0]) - atan2_f64(x * z, y * r);
       }
     } else {
+      r = sqrt(r2);
       t[0] = atan2(x * y, z * r);
     }
     t[1] = lg(fmax(y + r, DBL_EPSILON));
