@@ -298,6 +298,10 @@ jgm_status jgm_set_mesh(jgm_context* ctx, size_t nx, size_t ny, size_t nz, const
     for (size_t i = 0; i < n[a]; ++i) w += s[a][i];
     width[a] = w;
   }
+  ctx->shared_corners = true;
+  for (int a = 0; a < 3; ++a)
+    for (size_t i = 0; i + 1 < n[a]; ++i)
+      if (c[a][i] + s[a][i] != c[a][i + 1]) ctx->shared_corners = false;
   ctx->xwidth = width[0];
   ctx->ywidth = width[1];
   ctx->zwidth = width[2];

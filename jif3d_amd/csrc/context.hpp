@@ -135,6 +135,9 @@ struct jgm_context {
   std::vector<double> xc, yc, zc;  // corner coordinates, n+1 each
   std::vector<double> xs, ys, zs;  // cell sizes, n each
   double xwidth = 0, ywidth = 0, zwidth = 0;
+  // every cell ends where the next one begins (coord[i] + size[i] == coord[i + 1] on every
+  // axis): neighbouring cells share their corners exactly
+  bool shared_corners = false;
   bool mesh_set = false;
   // device mesh: corner coordinates used by the corner-first kernels (n+1 each),
   // and the per-cell origin/size arrays used by the per-cell kernels.

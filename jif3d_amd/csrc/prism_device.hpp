@@ -18,6 +18,7 @@
 #include <hip/hip_runtime.h>
 #include <cfloat>
 #include <cstdint>
+#include <type_traits>
 
 #include "log_table.hpp"
 
@@ -96,6 +97,9 @@ __device__ __forceinline__ double log_pos_f64(double a) {
 struct LogPoly {
   __device__ __forceinline__ double operator()(double a) const { return log_pos_f64(a); }
 };
+
+// gz alone on the library's logarithm and arctangent (kMaskScalar only).
+struct LogLibrary {};
 
 // Logarithm of a normal a > 0 from a 256-entry table in LDS (Tang's table-driven method, ACM
 // TOMS 16, 1990, with the reduced argument formed by one FMA): a = 2^e m, m in [1/2, 1), the
@@ -264,7 +268,7 @@ __device__ __forceinline__ void corner_terms_f64(double x, double y, double z, d
     t[2] = lg(fmax(x + r, DBL_EPSILON));
     return;
   }
-  if constexpr (MASK == kMaskScalar) {
+  if constexpr (MASK == kMaskScalar && !std::is_same_v<Log, LogLibrary>) {
     // no zero coordinate, products of two offsets within atan2_f64's range, and arguments
     // of the logarithms where the guarded ones equal them
     const double r = sqrt_pos_f64(r2);
@@ -325,7 +329,7 @@ __device__ __forceinline__ void corner_terms_f64(double x, double y, double z, d
 template <int MASK>
 __host__ __device__ inline void comp_scales(double* s) {
   int k = 0;
-  if (MASK & kZcol) { s[k++] = kGravConst; s[k++] = -kGravConst; s[k++] = -kGravConst; }
+  if (MASK & (kZcol | kZder)) { s[k++] = kGravConst; s[k++] = -kGravConst; s[k++] = -kGravConst; }
   if (MASK & kGz) s[k++] = -kGravConst;
   if (MASK & kDiag) { s[k++] = kGravConst; s[k++] = kGravConst; s[k++] = kGravConst; }
   if (MASK & kOff) { s[k++] = -kGravConst; s[k++] = -kGravConst; s[k++] = -kGravConst; }
