@@ -12,6 +12,24 @@
 
 namespace jgm {
 
+// a + p[0] + p[stride] + ... + p[(n - 1) stride], added in that order.  The loads of 16 terms
+// are issued before the first is added: a lane that waits for each term in turn spends the
+// memory latency n times (100 partial sums of 4851 corners: 24 us one by one, 8 us with eight
+// in flight, 6 us with 16).
+__device__ __forceinline__ double sum_strided(double a, const double* __restrict__ p, int n,
+                                              long stride) {
+  constexpr int U = 16;
+  for (int c = 0; c < n; c += U) {
+    double v[U];
+#pragma unroll
+    for (int u = 0; u < U; ++u) v[u] = p[(long)(c + u < n ? c + u : n - 1) * stride];
+#pragma unroll
+    for (int u = 0; u < U; ++u)
+      if (c + u < n) a += v[u];
+  }
+  return a;
+}
+
 struct FieldDir {
   double bx, by, bz, scale;  // direction cosines and F / (4 pi G)
 };

@@ -276,9 +276,7 @@ __global__ __launch_bounds__(kBlock) void k_sum_chunks(const double* __restrict_
                                                        double* __restrict__ out) {
   const long q = (long)blockIdx.x * blockDim.x + threadIdx.x;
   if (q >= n) return;
-  double a = 0.0;
-  for (int c = 0; c < nchunks; ++c) a += part[(long)c * n + q];
-  out[q] = a;
+  out[q] = sum_strided(0.0, part + q, nchunks, n);
 }
 
 // First pass of the chunk reduction: group g sums chunks [g per, (g + 1) per) of every
@@ -290,9 +288,7 @@ __global__ __launch_bounds__(kBlock) void k_sum_chunk_groups(const double* __res
   if (q >= n) return;
   const int c0 = (int)blockIdx.y * per;
   const int c1 = c0 + per < nchunks ? c0 + per : nchunks;
-  double a = 0.0;
-  for (int c = c0; c < c1; ++c) a += part[(long)c * n + q];
-  grp[(long)blockIdx.y * n + q] = a;
+  grp[(long)blockIdx.y * n + q] = sum_strided(0.0, part + (long)c0 * n + q, c1 - c0, n);
 }
 
 // g_c = 2 sum_{a,b,c} sigma(a,b,c) H(i+a, j+b, k+c)

@@ -35,12 +35,15 @@ __device__ inline double block_sum(double v, double* red) {
   return r;
 }
 
-// w(I,J,K) = sum sigma rho over the eight cells sharing the corner (rho zero outside)
+// w(I,J,K) = sum sigma rho over the eight cells sharing the corner (rho zero outside); clears
+// the error that the samples' kernel raises
 __global__ __launch_bounds__(kBlock) void k_check_weights(const double* __restrict__ rho,
                                                           int nx, int ny, int nz,
-                                                          double* __restrict__ w) {
+                                                          double* __restrict__ w,
+                                                          double* __restrict__ err) {
   const long ncx = nx + 1, ncy = ny + 1, ncz = nz + 1;
   const long q = (long)blockIdx.x * blockDim.x + threadIdx.x;
+  if (q == 0) err[0] = 0.0;
   if (q >= ncx * ncy * ncz) return;
   const int K = (int)(q % ncz);
   const long t = q / ncz;
@@ -58,16 +61,39 @@ __global__ __launch_bounds__(kBlock) void k_check_weights(const double* __restri
   w[q] = acc;
 }
 
+// Survey maximum of |raw| of one raw component, by one workgroup
+__device__ inline void survey_max(const double* __restrict__ raw, int S, int kraw, int m,
+                                  double* red, double* __restrict__ smax) {
+  double v = 0.0;
+  for (int s = threadIdx.x; s < S; s += blockDim.x) v = fmax(v, fabs(raw[(long)s * kraw + m]));
+  red[threadIdx.x] = v;
+  __syncthreads();
+  for (int w = blockDim.x / 2; w > 0; w >>= 1) {
+    if ((int)threadIdx.x < w) red[threadIdx.x] = fmax(red[threadIdx.x], red[threadIdx.x + w]);
+    __syncthreads();
+  }
+  if (threadIdx.x == 0) smax[m] = red[0];
+  __syncthreads();
+}
+
 // Forward at F sample sites: block (x, f) sums w(q) F_m(s_f, q) over a strided share of
-// the corners; partial[(x F + f) NC + m].
+// the corners; partial[(x F + f) NC + m].  The last row of blocks (y = F) takes the survey
+// maxima of the mixed raw data's components, which need nothing of the other rows.
 template <int MASK>
 __global__ __launch_bounds__(kBlock) void k_check_forward(
     const double* __restrict__ sx, const double* __restrict__ sy, const double* __restrict__ sz,
     const int* __restrict__ sidx, int F, const double* __restrict__ Xc,
     const double* __restrict__ Yc, const double* __restrict__ Zc, int ncy, int ncz, long nq,
-    const double* __restrict__ w, double* __restrict__ partial) {
+    const double* __restrict__ w, const double* __restrict__ raw, int S, int kraw,
+    double* __restrict__ smax, double* __restrict__ partial) {
   constexpr int NC = Ncomp<MASK>::value;
-  __shared__ double red[kBlock / 64];
+  __shared__ double red[kBlock];
+  __shared__ LogTableShared tab;
+  if ((int)blockIdx.y == F) {
+    for (int m = blockIdx.x; m < kraw; m += gridDim.x) survey_max(raw, S, kraw, m, red, smax);
+    return;
+  }
+  const LogTable lg = tab.fill();
   const long stride = (long)gridDim.x * blockDim.x;
   const int f = blockIdx.y;
   const int s = sidx[f];
@@ -81,7 +107,7 @@ __global__ __launch_bounds__(kBlock) void k_check_forward(
     const int J = (int)(t % ncy);
     const int I = (int)(t / ncy);
     double tv[NC];
-    corner_terms_f64<MASK>(px - Xc[I], py - Yc[J], pz - Zc[K], tv);
+    corner_terms_f64<MASK>(px - Xc[I], py - Yc[J], pz - Zc[K], tv, lg);
     const double wq = w[q];
 #pragma unroll
     for (int m = 0; m < NC; ++m) acc[m] = fma(wq, tv[m], acc[m]);
@@ -93,43 +119,28 @@ __global__ __launch_bounds__(kBlock) void k_check_forward(
   }
 }
 
-// Survey maximum of |raw| per raw component: block m writes smax[m]
-__global__ __launch_bounds__(kBlock) void k_check_survey_max(const double* __restrict__ raw,
-                                                             int S, int kraw,
-                                                             double* __restrict__ smax) {
-  __shared__ double red[kBlock];
-  const int m = blockIdx.x;
-  double v = 0.0;
-  for (int s = threadIdx.x; s < S; s += blockDim.x) v = fmax(v, fabs(raw[(long)s * kraw + m]));
-  red[threadIdx.x] = v;
-  __syncthreads();
-  for (int w = blockDim.x / 2; w > 0; w >>= 1) {
-    if ((int)threadIdx.x < w) red[threadIdx.x] = fmax(red[threadIdx.x], red[threadIdx.x + w]);
-    __syncthreads();
-  }
-  if (threadIdx.x == 0) smax[m] = red[0];
-}
-
 // FP64 raw data of sample site f (block f: the block partials summed as a tree, then
 // background and assembly as the forward) against the mixed raw data;
-// errs[f] = largest |difference| / survey maximum of its component.
+// err[0] = the largest |difference| / survey maximum of its component over all samples (the
+// errors are not negative, so their bit patterns order as they do).
 template <int MASK>
 __global__ __launch_bounds__(kBlock) void k_check_forward_sites(
     const double* __restrict__ partial, int nblocks, const int* __restrict__ sidx, int F,
     const double* __restrict__ bgT, const double* __restrict__ bgvals, int L, int kind,
     FieldDir fd, const double* __restrict__ mixed_raw, const double* __restrict__ smax,
-    double* __restrict__ errs) {
+    unsigned long long* __restrict__ err) {
   constexpr int NC = Ncomp<MASK>::value;
   __shared__ double red[kBlock / 64];
   const int f = blockIdx.x;
   double acc[NC], sc[NC];
   comp_scales<MASK>(sc);
 #pragma unroll
-  for (int m = 0; m < NC; ++m) {
-    double a = 0.0;
-    for (int b = threadIdx.x; b < nblocks; b += blockDim.x) a += partial[((long)b * F + f) * NC + m];
-    acc[m] = block_sum(a, red) * sc[m];
-  }
+  for (int m = 0; m < NC; ++m) acc[m] = 0.0;
+  for (int b = threadIdx.x; b < nblocks; b += blockDim.x)
+#pragma unroll
+    for (int m = 0; m < NC; ++m) acc[m] += partial[((long)b * F + f) * NC + m];
+#pragma unroll
+  for (int m = 0; m < NC; ++m) acc[m] = block_sum(acc[m], red) * sc[m];
   if (threadIdx.x != 0) return;
   double u[7], raw[10];
   spread_components<MASK>(acc, u);
@@ -140,30 +151,14 @@ __global__ __launch_bounds__(kBlock) void k_check_forward_sites(
     const double d = fabs(raw[m] - mixed_raw[(long)s * kraw + m]);
     e = fmax(e, d / fmax(smax[m], 1e-300));
   }
-  errs[f] = e;
+  atomicMax(err, (unsigned long long)__double_as_longlong(e));
 }
 
-// out[0] = max of v[0..n).  One block.
-__global__ __launch_bounds__(kBlock) void k_check_max(const double* __restrict__ v, int n,
-                                                      double* __restrict__ out) {
-  __shared__ double red[kBlock];
+// max of |g| over block x of nb's grid-strided share of g[0..n)
+__device__ inline void grad_absmax(const double* __restrict__ g, long n, int x, int nb, double* red,
+                                   double* __restrict__ pm) {
   double e = 0.0;
-  for (int i = threadIdx.x; i < n; i += blockDim.x) e = fmax(e, v[i]);
-  red[threadIdx.x] = e;
-  __syncthreads();
-  for (int w = blockDim.x / 2; w > 0; w >>= 1) {
-    if ((int)threadIdx.x < w) red[threadIdx.x] = fmax(red[threadIdx.x], red[threadIdx.x + w]);
-    __syncthreads();
-  }
-  if (threadIdx.x == 0) out[0] = red[0];
-}
-
-// pm[block] = max of |g| over a grid-strided share of g[0..n)
-__global__ __launch_bounds__(kBlock) void k_check_absmax(const double* __restrict__ g, long n,
-                                                         double* __restrict__ pm) {
-  __shared__ double red[kBlock];
-  double e = 0.0;
-  for (long i = (long)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += (long)gridDim.x * blockDim.x)
+  for (long i = (long)x * blockDim.x + threadIdx.x; i < n; i += (long)nb * blockDim.x)
     e = fmax(e, fabs(g[i]));
   red[threadIdx.x] = e;
   __syncthreads();
@@ -171,37 +166,57 @@ __global__ __launch_bounds__(kBlock) void k_check_absmax(const double* __restric
     if ((int)threadIdx.x < w) red[threadIdx.x] = fmax(red[threadIdx.x], red[threadIdx.x + w]);
     __syncthreads();
   }
-  if (threadIdx.x == 0) pm[blockIdx.x] = red[0];
+  if (threadIdx.x == 0) pm[x] = red[0];
 }
 
-// Adjoint at FC sample cells: blocks (cell, split), threads over the split's sites,
-// g_c = 2 sum_s sum_m c_m(s) J_m(s, c) with the FP64 box term of the cell (the gridded
-// part; the background gradient is exact in both paths); gs[cell gridDim.y + split].
+// Adjoint at FC sample cells: block x < FC nsplit takes split x % nsplit of cell x / nsplit,
+// eight lanes per site, one for each corner of the cell,
+// g_c = 2 sum_s sum_m c_m(s) sum_corners sigma F_m (the gridded part; the background gradient
+// is exact in both paths); gs[cell nsplit + split].  The other nb blocks take the largest
+// |gradient| of their share.
 template <int MASK>
 __global__ __launch_bounds__(kBlock) void k_check_adjoint(
     const double* __restrict__ sx, const double* __restrict__ sy, const double* __restrict__ sz,
     int S, const double* __restrict__ rm, int kind, FieldDir fd, const int* __restrict__ cidx,
     const double* __restrict__ xlo, const double* __restrict__ ylo,
     const double* __restrict__ zlo, const double* __restrict__ xsz,
-    const double* __restrict__ ysz, const double* __restrict__ zsz, int ny, int nz,
+    const double* __restrict__ ysz, const double* __restrict__ zsz, int ny, int nz, int FC,
+    int nsplit, const double* __restrict__ grad, long N, int nb, double* __restrict__ pm,
     double* __restrict__ gs) {
   constexpr int NC = Ncomp<MASK>::value;
   __shared__ double red[kBlock];
-  const long c = cidx[blockIdx.x];
+  __shared__ LogTableShared tab;
+  const int x = (int)blockIdx.x - FC * nsplit;
+  if (x >= 0) {
+    grad_absmax(grad, N, x, nb, red, pm);
+    return;
+  }
+  const LogTable lg = tab.fill();
+  const int f = blockIdx.x / nsplit, split = blockIdx.x % nsplit;
+  const long c = cidx[f];
   const int k = (int)(c % nz);
   const long t = c / nz;
   const int j = (int)(t % ny);
   const int i = (int)(t / ny);
+  const int a = threadIdx.x & 1, b = (threadIdx.x >> 1) & 1, d = (threadIdx.x >> 2) & 1;
+  const double cx = a ? xlo[i] + xsz[i] : xlo[i], cy = b ? ylo[j] + ysz[j] : ylo[j];
+  const double cz = d ? zlo[k] + zsz[k] : zlo[k];
+  double sc[NC];
+  comp_scales<MASK>(sc);
   double acc = 0.0;
-  for (int s = blockIdx.y * blockDim.x + threadIdx.x; s < S; s += gridDim.y * blockDim.x) {
+  for (int s = split * (kBlock / 8) + (int)(threadIdx.x >> 3); s < S; s += nsplit * (kBlock / 8)) {
     double v[NC], u[7], c7[7];
-    box_terms_f64<MASK>(sx[s], sy[s], sz[s], xlo[i], ylo[j], zlo[k], xsz[i], ysz[j], zsz[k], v);
+    corner_terms_f64<MASK>(sx[s] - cx, sy[s] - cy, sz[s] - cz, v, lg);
+#pragma unroll
+    for (int m = 0; m < NC; ++m) v[m] *= sc[m];
     spread_components<MASK>(v, u);
     site_coefficients(rm, s, kind, fd, c7);
-    for (int m = 0; m < 7; ++m) acc = fma(c7[m], u[m], acc);
+    double h = 0.0;
+    for (int m = 0; m < 7; ++m) h = fma(c7[m], u[m], h);
+    acc += ((a + b + d) & 1) ? h : -h;
   }
   const double g = block_sum(acc, red);
-  if (threadIdx.x == 0) gs[(long)blockIdx.x * gridDim.y + blockIdx.y] = 2.0 * g;
+  if (threadIdx.x == 0) gs[blockIdx.x] = 2.0 * g;
 }
 
 // err[0] = max over sample cells |g_mixed - g_fp64| / max over cells |g_mixed| (the latter
@@ -226,8 +241,7 @@ __global__ __launch_bounds__(kBlock) void k_check_adjoint_finish(const double* _
   __syncthreads();
   double e = 0.0;
   for (int f = threadIdx.x; f < FC; f += blockDim.x) {
-    double g = 0.0;
-    for (int q = 0; q < nsplit; ++q) g += gs[(long)f * nsplit + q];
+    const double g = sum_strided(0.0, gs + (long)f * nsplit, nsplit, 1);
     e = fmax(e, fabs(grad[cidx[f]] - g) / fmax(gmax, 1e-300));
   }
   red[threadIdx.x] = e;
@@ -284,37 +298,36 @@ hipError_t check_forward_impl(jgm_context* ctx, int kind, const double* model,
   const int kraw = (int)raw_per_site(kind);
   const int ncy = (int)ctx->ny + 1, ncz = (int)ctx->nz + 1;
   const long nq = (long)ncorners(ctx);
-  // blocks per sample site: about 2 CUs' worth over all sites, each thread taking at least
-  // 8 corners so that the block sums stay a small part of the work (on small meshes a floor
-  // of 32 left most CUs idle: config 1's 139K corners gave 17 blocks per site)
-  const long want = std::max<long>(1, 2L * ctx->cu_count / std::max(1, F));
-  const int nblocks = (int)std::max<long>(1, std::min<long>(want, (nq + 8L * kBlock - 1) / (8L * kBlock)));
+  // blocks per sample site: about 8 per CU over all sites (two waves per SIMD, as 2 blocks per
+  // CU gave, leave the FP64 chains' latency in the open: the whole check of 1.08M corners takes
+  // 95 us with 2, 70 us with 8),
+  // each thread taking at least 2 corners so that the block sums stay a small part of the work
+  // (on small meshes a higher floor leaves CUs idle: 139K corners ran 17 us with 8, 12 us with 2)
+  const long want = std::max<long>(1, 8L * ctx->cu_count / std::max(1, F));
+  const int nblocks = (int)std::max<long>(1, std::min<long>(want, (nq + 2L * kBlock - 1) / (2L * kBlock)));
   hipError_t e;
-  // partials (nblocks F NC), survey maxima (kraw), per-site errors (F), the error (1)
+  // partials (nblocks F NC), survey maxima (kraw), the error (1)
   if ((e = ctx->check_w.ensure(sizeof(double) * (size_t)nq)) != hipSuccess ||
-      (e = ctx->check_part.ensure(sizeof(double) * ((size_t)nblocks * F * NC + kraw + F + 1))) !=
+      (e = ctx->check_part.ensure(sizeof(double) * ((size_t)nblocks * F * NC + kraw + 1))) !=
           hipSuccess)
     return e;
   double* part = ctx->check_part.as<double>();
   double* smax = part + (size_t)nblocks * F * NC;
-  double* errs = smax + kraw;
-  double* err = errs + F;
+  double* err = smax + kraw;
   {
     ProfScope ps(ctx, "mixed_check_forward_fp64");
     hipLaunchKernelGGL(k_check_weights, dim3(blocks_for(nq)), dim3(kBlock), 0, st, model,
-                       (int)ctx->nx, (int)ctx->ny, (int)ctx->nz, ctx->check_w.as<double>());
-    hipLaunchKernelGGL((k_check_forward<MASK>), dim3(nblocks, F), dim3(kBlock), 0, st,
+                       (int)ctx->nx, (int)ctx->ny, (int)ctx->nz, ctx->check_w.as<double>(), err);
+    hipLaunchKernelGGL((k_check_forward<MASK>), dim3(nblocks, F + 1), dim3(kBlock), 0, st,
                        ctx->d_sx.as<const double>(), ctx->d_sy.as<const double>(),
                        ctx->d_sz.as<const double>(), ctx->check_sidx.as<const int>(), F,
                        ctx->d_Xc.as<const double>(), ctx->d_Yc.as<const double>(),
                        ctx->d_Zc.as<const double>(), ncy, ncz, nq,
-                       ctx->check_w.as<const double>(), part);
-    hipLaunchKernelGGL(k_check_survey_max, dim3(kraw), dim3(kBlock), 0, st, mixed_raw, S, kraw,
-                       smax);
+                       ctx->check_w.as<const double>(), mixed_raw, S, kraw, smax, part);
     hipLaunchKernelGGL((k_check_forward_sites<MASK>), dim3(F), dim3(kBlock), 0, st, part,
                        nblocks, ctx->check_sidx.as<const int>(), F, ctx->bgT.as<const double>(),
-                       model + N, L, kind, field_dir(ctx), mixed_raw, smax, errs);
-    hipLaunchKernelGGL(k_check_max, dim3(1), dim3(kBlock), 0, st, errs, F, err);
+                       model + N, L, kind, field_dir(ctx), mixed_raw, smax,
+                       reinterpret_cast<unsigned long long*>(err));
   }
   if ((e = hipGetLastError()) != hipSuccess) return e;
   if ((e = hipMemcpyAsync(err_host, err, sizeof(double), hipMemcpyDeviceToHost, st)) !=
@@ -329,7 +342,7 @@ hipError_t check_adjoint_impl(jgm_context* ctx, int kind, const double* raw_misf
   hipStream_t st = ctx->stream;
   const int FC = (int)ctx->check_FC;
   const long N = (long)ncells(ctx);
-  const int nsplit = (int)std::max<size_t>(1, std::min<size_t>(32, (ctx->S + kBlock - 1) / kBlock));
+  const int nsplit = (int)std::max<size_t>(1, std::min<size_t>(64, (ctx->S + kBlock / 8 - 1) / (kBlock / 8)));
   const int nb = (int)std::max<long>(1, std::min<long>(2L * ctx->cu_count, (N + kBlock - 1) / kBlock));
   hipError_t e;
   // per-split sums (FC nsplit), block maxima of |grad| (nb), the error (1)
@@ -340,14 +353,14 @@ hipError_t check_adjoint_impl(jgm_context* ctx, int kind, const double* raw_misf
   double* err = pm + nb;
   {
     ProfScope ps(ctx, "mixed_check_adjoint_fp64");
-    hipLaunchKernelGGL((k_check_adjoint<MASK>), dim3(FC, nsplit), dim3(kBlock), 0, st,
+    hipLaunchKernelGGL((k_check_adjoint<MASK>), dim3(FC * nsplit + nb), dim3(kBlock), 0, st,
                        ctx->d_sx.as<const double>(), ctx->d_sy.as<const double>(),
                        ctx->d_sz.as<const double>(), (int)ctx->S, raw_misfit, kind, field_dir(ctx),
                        ctx->check_cidx.as<const int>(), ctx->d_xlo.as<const double>(),
                        ctx->d_ylo.as<const double>(), ctx->d_zlo.as<const double>(),
                        ctx->d_xsz.as<const double>(), ctx->d_ysz.as<const double>(),
-                       ctx->d_zsz.as<const double>(), (int)ctx->ny, (int)ctx->nz, gs);
-    hipLaunchKernelGGL(k_check_absmax, dim3(nb), dim3(kBlock), 0, st, grad, N, pm);
+                       ctx->d_zsz.as<const double>(), (int)ctx->ny, (int)ctx->nz, FC, nsplit, grad,
+                       N, nb, pm, gs);
     hipLaunchKernelGGL(k_check_adjoint_finish, dim3(1), dim3(kBlock), 0, st, grad, pm, nb,
                        ctx->check_cidx.as<const int>(), gs, FC, nsplit, err);
   }

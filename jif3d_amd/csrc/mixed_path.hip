@@ -609,6 +609,8 @@ __global__ __launch_bounds__(kBlock) void k_near_forward(
     const double* __restrict__ Zc, const double* __restrict__ rho, int nx, int ny, int nz,
     double* __restrict__ nearout) {
   constexpr int NC = Ncomp<MASK>::value;
+  __shared__ LogTableShared tab;
+  const LogTable lg = tab.fill();
   const int s = blockIdx.x;
   const int i0 = box[s * 6 + 0], i1 = box[s * 6 + 1];
   const int j0 = box[s * 6 + 2], j1 = box[s * 6 + 3];
@@ -637,7 +639,7 @@ __global__ __launch_bounds__(kBlock) void k_near_forward(
             w += ((a + b + c) & 1) ? v : -v;
           }
       double t[NC];
-      corner_terms_f64<MASK>(px - Xc[I], py - Yc[J], pz - Zc[K], t);
+      corner_terms_f64<MASK>(px - Xc[I], py - Yc[J], pz - Zc[K], t, lg);
 #pragma unroll
       for (int m = 0; m < NC; ++m) acc[m] = fma(w, t[m], acc[m]);
     }
@@ -692,9 +694,8 @@ __global__ __launch_bounds__(kBlock) void k_mixed_forward_sums(const double* __r
   if (s >= S) return;
 #pragma unroll
   for (int m = 0; m < NC; ++m) {
-    double a = nearout[(long)s * NC + m];
-    for (int c = 0; c < nchunks; ++c) a += farpart[((long)c * NC + m) * S + s];
-    sums[(long)s * NC + m] = a;
+    sums[(long)s * NC + m] =
+        sum_strided(nearout[(long)s * NC + m], farpart + (long)m * S + s, nchunks, (long)NC * S);
   }
 }
 
@@ -1011,6 +1012,8 @@ __global__ __launch_bounds__(kBlock) void k_near_adjoint_site(
     const long* __restrict__ cell_off, double* __restrict__ hbuf,
     double* __restrict__ vbuf) {
   constexpr int NC = Ncomp<MASK>::value;
+  __shared__ LogTableShared tab;
+  const LogTable lg = tab.fill();
   const int s = blockIdx.x;
   const int i0 = box[s * 6 + 0], i1 = box[s * 6 + 1];
   const int j0 = box[s * 6 + 2], j1 = box[s * 6 + 3];
@@ -1027,7 +1030,7 @@ __global__ __launch_bounds__(kBlock) void k_near_adjoint_site(
     const int J = j0 + (q / ck) % cj;
     const int I = i0 + q / (ck * cj);
     double t[NC];
-    corner_terms_f64<MASK>(px - Xc[I], py - Yc[J], pz - Zc[K], t);
+    corner_terms_f64<MASK>(px - Xc[I], py - Yc[J], pz - Zc[K], t, lg);
     double h = 0.0;
 #pragma unroll
     for (int m = 0; m < NC; ++m) h = fma(cs[m], t[m], h);
@@ -1086,8 +1089,19 @@ __global__ __launch_bounds__(64) void k_near_adjoint_gather(
       }
       __syncthreads();
       if (k <= kmax)
-        for (int q = 0; q < np; ++q)
-          if (k >= sk0[q] && k <= sk1[q]) acc += vbuf[soff[q] + k];
+        for (int q0 = 0; q0 < np; q0 += 8) {  // eight loads in flight, added in site order
+          double v[8];
+          bool in[8];
+#pragma unroll
+          for (int u = 0; u < 8; ++u) {
+            const int q = min(q0 + u, np - 1);
+            in[u] = q0 + u < np && k >= sk0[q] && k <= sk1[q];
+            v[u] = in[u] ? vbuf[soff[q] + k] : 0.0;
+          }
+#pragma unroll
+          for (int u = 0; u < 8; ++u)
+            if (in[u]) acc += v[u];
+        }
     }
     if (k <= kmax) gnear[((long)i * ny + j) * nz + k] = acc;
   }
@@ -1108,9 +1122,7 @@ __global__ __launch_bounds__(kBlock) void k_adjoint_mixed_finish(const double* _
     grad[c] = 0.0;
     return;
   }
-  double a = gnear[c];
-  for (int q = 0; q < nchunks; ++q) a += gpart[(long)q * n + c];
-  grad[c] = a;
+  grad[c] = sum_strided(gnear[c], gpart + c, nchunks, n);
 }
 
 int mask_of(int kind) {

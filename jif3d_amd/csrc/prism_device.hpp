@@ -244,8 +244,8 @@ __device__ __forceinline__ void corner_terms_f64(double x, double y, double z, d
     t[0] = (fmin(fmin(fabs(x), fabs(y)), fabs(z)) >= 1e-140 && r >= DBL_EPSILON && r <= 1e140)
                ? atan2_f64(x * y, z * r)
                : atan2(x * y, z * r);
-    t[1] = log_pos_f64(fmax(y + r, DBL_EPSILON));
-    t[2] = log_pos_f64(fmax(x + r, DBL_EPSILON));
+    t[1] = lg(fmax(y + r, DBL_EPSILON));
+    t[2] = lg(fmax(x + r, DBL_EPSILON));
     return;
   }
   if constexpr (MASK == kMaskZder) {
