@@ -132,43 +132,72 @@ size_t data_per_site(const jgm_context* ctx, int kind) {
   return ctx->transform == JGM_TF_NONE ? jgm::raw_per_site(kind) : 1;
 }
 
-// Host-memory form of a device entry point: copies the inputs into temporary device
-// buffers, runs `call` on their device pointers, copies the outputs back and waits.
+// Host-memory form of a device entry point: copies the inputs to device buffers, runs `call`
+// on their device pointers, copies the outputs back and waits.  The device buffers are the
+// context's, kept between calls, up to kStageKept bytes a call (larger ones are given back when
+// the call ends); up to kStagePinned bytes the copies pass through the context's page-locked
+// memory, with one wait at the end instead of one for each copy of pageable memory.  Data and
+// gradient of 4000 cells and 100 sites: 175 us with an allocation and pageable copies, 136 us.
 struct HostArg {
   const double* in;  // host input (or nullptr)
   double* out;       // host output (or nullptr)
   size_t n;          // doubles
 };
+constexpr size_t kStageKept = (size_t)512 << 20, kStagePinned = (size_t)4 << 20;
+
 template <size_t NA, class F>
 jgm_status run_staged(jgm_context* ctx, const char* where, const HostArg (&args)[NA], F call) {
-  jgm::DeviceBuffer buf[NA];
+  static_assert(NA <= sizeof(ctx->host_stage) / sizeof(ctx->host_stage[0]), "staging buffers");
+  size_t total = 0;
+  for (size_t a = 0; a < NA; ++a) total += sizeof(double) * args[a].n;
+  hipError_t e = hipSuccess;
+  const bool kept = total <= kStageKept;
+  bool pinned = total <= kStagePinned;
+  if (pinned && !ctx->host_pin &&
+      hipHostMalloc(&ctx->host_pin, kStagePinned, hipHostMallocDefault) != hipSuccess) {
+    (void)hipGetLastError();  // no page-locked memory: copy from the caller's
+    ctx->host_pin = nullptr;
+    pinned = false;
+  }
+  jgm::DeviceBuffer own[NA];
   const double* dev_in[NA];
   double* dev_out[NA];
-  hipError_t e = hipSuccess;
+  double* pin[NA];
+  size_t used = 0;
   for (size_t a = 0; a < NA && e == hipSuccess; ++a) {
     dev_in[a] = nullptr;
     dev_out[a] = nullptr;
+    pin[a] = pinned ? static_cast<double*>(ctx->host_pin) + used : nullptr;
+    used += args[a].n;
     if (!args[a].in && !args[a].out) continue;
-    e = buf[a].ensure(sizeof(double) * (args[a].n ? args[a].n : 1));
-    if (e == hipSuccess && args[a].in && args[a].n)
-      e = hipMemcpyAsync(buf[a].ptr, args[a].in, sizeof(double) * args[a].n,
-                         hipMemcpyHostToDevice, ctx->stream);
-    dev_in[a] = static_cast<const double*>(buf[a].ptr);
-    dev_out[a] = static_cast<double*>(buf[a].ptr);
+    const size_t bytes = sizeof(double) * args[a].n;
+    jgm::DeviceBuffer& buf = kept ? ctx->host_stage[a] : own[a];
+    e = buf.ensure(bytes ? bytes : sizeof(double));
+    if (e == hipSuccess && args[a].in && bytes) {
+      if (pinned) std::memcpy(pin[a], args[a].in, bytes);
+      e = hipMemcpyAsync(buf.ptr, pinned ? pin[a] : args[a].in, bytes, hipMemcpyHostToDevice,
+                         ctx->stream);
+    }
+    dev_in[a] = static_cast<const double*>(buf.ptr);
+    dev_out[a] = static_cast<double*>(buf.ptr);
   }
   jgm_status st = JGM_OK;
   if (e == hipSuccess) {
     st = call(dev_in, dev_out);
     for (size_t a = 0; a < NA && st == JGM_OK && e == hipSuccess; ++a)
       if (args[a].out && args[a].n)
-        e = hipMemcpyAsync(args[a].out, buf[a].ptr, sizeof(double) * args[a].n,
+        e = hipMemcpyAsync(pinned ? pin[a] : args[a].out, dev_out[a], sizeof(double) * args[a].n,
                            hipMemcpyDeviceToHost, ctx->stream);
   }
   hipError_t e2 = hipStreamSynchronize(ctx->stream);
-  for (size_t a = 0; a < NA; ++a) buf[a].release();
+  for (size_t a = 0; a < NA; ++a) own[a].release();
   if (st != JGM_OK) return st;
   if (e != hipSuccess) return hip_fail(e, where);
   if (e2 != hipSuccess) return hip_fail(e2, where);
+  if (pinned)
+    for (size_t a = 0; a < NA; ++a)
+      if (args[a].out && args[a].n)
+        std::memcpy(args[a].out, pin[a], sizeof(double) * args[a].n);
   return JGM_OK;
 }
 
@@ -219,8 +248,8 @@ jgm_status jgm_destroy(jgm_context* ctx) {
                                &ctx->d_zlo, &ctx->d_xsz, &ctx->d_ysz, &ctx->d_zsz, &ctx->d_sx,
                                &ctx->d_sy, &ctx->d_sz, &ctx->bgT, &ctx->near.box,
                                &ctx->weights, &ctx->partial, &ctx->raw,
-                               &ctx->coef, &ctx->hpart, &ctx->hsum, &ctx->model_stage,
-                               &ctx->out_stage, &ctx->misfit_stage, &ctx->grad_stage,
+                               &ctx->coef, &ctx->hpart, &ctx->hsum,
+                               &ctx->out_stage, &ctx->misfit_stage,
                                &ctx->farpart, &ctx->nearpart, &ctx->coef32, &ctx->storedJ, &ctx->storedJ_vec,
                                &ctx->storedJ_bf16, &ctx->storedJ_bf16c, &ctx->storedJ_rhs16lo,
                                &ctx->near.col_ptr, &ctx->near.col_sites, &ctx->near.col_ids,
@@ -232,6 +261,8 @@ jgm_status jgm_destroy(jgm_context* ctx) {
                                &ctx->near.listed, &ctx->acc64, &ctx->raw_cache_model, &ctx->raw_cache_raw, &ctx->raw_cache_flag,
                                &ctx->partsum, &ctx->chunk_scratch, &ctx->mag_part};
   for (auto* b : bufs) b->release();
+  for (auto& b : ctx->host_stage) b.release();
+  if (ctx->host_pin) (void)hipHostFree(ctx->host_pin);
   jgm::release_slab_mesh(ctx);
   jgm::release_host_storedj(ctx);
   if (ctx->copy_stream) (void)hipStreamDestroy(ctx->copy_stream);
@@ -585,23 +616,11 @@ jgm_status jgm_forward_host(jgm_context* ctx, jgm_kind kind, jgm_precision prec,
   if (st != JGM_OK) return st;
   if (!model || !out) return fail(JGM_ERR_INVALID_ARGUMENT, "null model or output pointer");
   DeviceGuard g(ctx->device);
-  const size_t np = jgm::nparams(ctx, kind);
-  const size_t nout = ctx->S * data_per_site(ctx, kind);
-  hipError_t e;
-  if ((e = ctx->model_stage.ensure(sizeof(double) * (np ? np : 1))) != hipSuccess)
-    return hip_fail(e, "forward_host");
-  if ((e = ctx->grad_stage.ensure(sizeof(double) * (nout ? nout : 1))) != hipSuccess)
-    return hip_fail(e, "forward_host");
-  if (np && (e = hipMemcpyAsync(ctx->model_stage.ptr, model, sizeof(double) * np,
-                                hipMemcpyHostToDevice, ctx->stream)) != hipSuccess)
-    return hip_fail(e, "forward_host");
-  st = jgm_forward(ctx, kind, prec, ctx->model_stage.as<double>(), ctx->grad_stage.as<double>());
-  if (st != JGM_OK) return st;
-  if (nout && (e = hipMemcpyAsync(out, ctx->grad_stage.ptr, sizeof(double) * nout,
-                                  hipMemcpyDeviceToHost, ctx->stream)) != hipSuccess)
-    return hip_fail(e, "forward_host");
-  if ((e = hipStreamSynchronize(ctx->stream)) != hipSuccess) return hip_fail(e, "forward_host");
-  return JGM_OK;
+  const HostArg args[2] = {{model, nullptr, jgm::nparams(ctx, kind)},
+                           {nullptr, out, ctx->S * data_per_site(ctx, kind)}};
+  return run_staged(ctx, "forward_host", args, [&](const double* const* in, double* const* o) {
+    return jgm_forward(ctx, kind, prec, in[0], o[1]);
+  });
 }
 
 jgm_status jgm_adjoint_host(jgm_context* ctx, jgm_kind kind, jgm_precision prec,
@@ -611,37 +630,12 @@ jgm_status jgm_adjoint_host(jgm_context* ctx, jgm_kind kind, jgm_precision prec,
   if (!misfit || !grad) return fail(JGM_ERR_INVALID_ARGUMENT, "null misfit or gradient pointer");
   DeviceGuard g(ctx->device);
   const size_t np = jgm::nparams(ctx, kind);
-  const size_t nmis = ctx->S * data_per_site(ctx, kind);
-  jgm::DeviceBuffer dmis;  // separate from the internal misfit_stage used by transforms
-  hipError_t e;
-  if ((e = ctx->model_stage.ensure(sizeof(double) * (np ? np : 1))) != hipSuccess)
-    return hip_fail(e, "adjoint_host");
-  if ((e = ctx->grad_stage.ensure(sizeof(double) * (np ? np : 1))) != hipSuccess)
-    return hip_fail(e, "adjoint_host");
-  if ((e = dmis.ensure(sizeof(double) * (nmis ? nmis : 1))) != hipSuccess)
-    return hip_fail(e, "adjoint_host");
-  if (model && np &&
-      (e = hipMemcpyAsync(ctx->model_stage.ptr, model, sizeof(double) * np, hipMemcpyHostToDevice,
-                          ctx->stream)) != hipSuccess) {
-    dmis.release();
-    return hip_fail(e, "adjoint_host");
-  }
-  if (nmis && (e = hipMemcpyAsync(dmis.ptr, misfit, sizeof(double) * nmis, hipMemcpyHostToDevice,
-                                  ctx->stream)) != hipSuccess) {
-    dmis.release();
-    return hip_fail(e, "adjoint_host");
-  }
-  st = jgm_adjoint(ctx, kind, prec, model ? ctx->model_stage.as<double>() : nullptr,
-                   dmis.as<double>(), ctx->grad_stage.as<double>());
-  if (st == JGM_OK && np)
-    e = hipMemcpyAsync(grad, ctx->grad_stage.ptr, sizeof(double) * np, hipMemcpyDeviceToHost,
-                       ctx->stream);
-  hipError_t e2 = hipStreamSynchronize(ctx->stream);
-  dmis.release();
-  if (st != JGM_OK) return st;
-  if (e != hipSuccess) return hip_fail(e, "adjoint_host");
-  if (e2 != hipSuccess) return hip_fail(e2, "adjoint_host");
-  return JGM_OK;
+  const HostArg args[3] = {{model, nullptr, model ? np : 0},
+                           {misfit, nullptr, ctx->S * data_per_site(ctx, kind)},
+                           {nullptr, grad, np}};
+  return run_staged(ctx, "adjoint_host", args, [&](const double* const* in, double* const* o) {
+    return jgm_adjoint(ctx, kind, prec, model ? in[0] : nullptr, in[1], o[2]);
+  });
 }
 
 jgm_status jgm_forward_batch(jgm_context* ctx, jgm_kind kind, jgm_precision prec, size_t nmodels,
@@ -1079,24 +1073,12 @@ jgm_status jgm_storedj_forward_host(jgm_context* ctx, jgm_gemm_precision prec,
   if (st != JGM_OK) return st;
   if (!model || !out) return fail(JGM_ERR_INVALID_ARGUMENT, "null model or output pointer");
   DeviceGuard g(ctx->device);
-  const size_t np = jgm::nparams(ctx, ctx->storedJ_kind);
-  const size_t nout = ctx->S * data_per_site(ctx, ctx->storedJ_kind);
-  hipError_t e;
-  if ((e = ctx->model_stage.ensure(sizeof(double) * (np ? np : 1))) != hipSuccess)
-    return hip_fail(e, "storedj_forward_host");
-  if ((e = ctx->grad_stage.ensure(sizeof(double) * (nout ? nout : 1))) != hipSuccess)
-    return hip_fail(e, "storedj_forward_host");
-  if ((e = hipMemcpyAsync(ctx->model_stage.ptr, model, sizeof(double) * np,
-                          hipMemcpyHostToDevice, ctx->stream)) != hipSuccess)
-    return hip_fail(e, "storedj_forward_host");
-  st = jgm_storedj_forward(ctx, prec, ctx->model_stage.as<double>(), ctx->grad_stage.as<double>());
-  if (st != JGM_OK) return st;
-  if (nout && (e = hipMemcpyAsync(out, ctx->grad_stage.ptr, sizeof(double) * nout,
-                                  hipMemcpyDeviceToHost, ctx->stream)) != hipSuccess)
-    return hip_fail(e, "storedj_forward_host");
-  if ((e = hipStreamSynchronize(ctx->stream)) != hipSuccess)
-    return hip_fail(e, "storedj_forward_host");
-  return JGM_OK;
+  const HostArg args[2] = {{model, nullptr, jgm::nparams(ctx, ctx->storedJ_kind)},
+                           {nullptr, out, ctx->S * data_per_site(ctx, ctx->storedJ_kind)}};
+  return run_staged(ctx, "storedj_forward_host", args,
+                    [&](const double* const* in, double* const* o) {
+                      return jgm_storedj_forward(ctx, prec, in[0], o[1]);
+                    });
 }
 
 jgm_status jgm_storedj_gradient_host(jgm_context* ctx, jgm_gemm_precision prec,
@@ -1106,36 +1088,13 @@ jgm_status jgm_storedj_gradient_host(jgm_context* ctx, jgm_gemm_precision prec,
   if (!misfit || !grad) return fail(JGM_ERR_INVALID_ARGUMENT, "null misfit or gradient pointer");
   DeviceGuard g(ctx->device);
   const size_t np = jgm::nparams(ctx, ctx->storedJ_kind);
-  const size_t nmis = ctx->S * data_per_site(ctx, ctx->storedJ_kind);
-  jgm::DeviceBuffer dmis;  // separate from the internal misfit_stage used by transforms
-  hipError_t e = hipSuccess;
-  if ((e = ctx->model_stage.ensure(sizeof(double) * (np ? np : 1))) != hipSuccess)
-    return hip_fail(e, "storedj_gradient_host");
-  if ((e = ctx->grad_stage.ensure(sizeof(double) * (np ? np : 1))) != hipSuccess)
-    return hip_fail(e, "storedj_gradient_host");
-  if ((e = dmis.ensure(sizeof(double) * (nmis ? nmis : 1))) != hipSuccess)
-    return hip_fail(e, "storedj_gradient_host");
-  if (model && (e = hipMemcpyAsync(ctx->model_stage.ptr, model, sizeof(double) * np,
-                                   hipMemcpyHostToDevice, ctx->stream)) != hipSuccess) {
-    dmis.release();
-    return hip_fail(e, "storedj_gradient_host");
-  }
-  if (nmis && (e = hipMemcpyAsync(dmis.ptr, misfit, sizeof(double) * nmis, hipMemcpyHostToDevice,
-                                  ctx->stream)) != hipSuccess) {
-    dmis.release();
-    return hip_fail(e, "storedj_gradient_host");
-  }
-  st = jgm_storedj_gradient(ctx, prec, model ? ctx->model_stage.as<double>() : nullptr,
-                            dmis.as<double>(), ctx->grad_stage.as<double>());
-  if (st == JGM_OK)
-    e = hipMemcpyAsync(grad, ctx->grad_stage.ptr, sizeof(double) * np, hipMemcpyDeviceToHost,
-                       ctx->stream);
-  hipError_t e2 = hipStreamSynchronize(ctx->stream);
-  dmis.release();
-  if (st != JGM_OK) return st;
-  if (e != hipSuccess) return hip_fail(e, "storedj_gradient_host");
-  if (e2 != hipSuccess) return hip_fail(e2, "storedj_gradient_host");
-  return JGM_OK;
+  const HostArg args[3] = {{model, nullptr, model ? np : 0},
+                           {misfit, nullptr, ctx->S * data_per_site(ctx, ctx->storedJ_kind)},
+                           {nullptr, grad, np}};
+  return run_staged(ctx, "storedj_gradient_host", args,
+                    [&](const double* const* in, double* const* o) {
+                      return jgm_storedj_gradient(ctx, prec, model ? in[0] : nullptr, in[1], o[2]);
+                    });
 }
 
 jgm_status jgm_storedj_release(jgm_context* ctx) {

@@ -213,9 +213,13 @@ struct jgm_context {
   jgm::NearBoxes near;
 
   // scratch
-  jgm::DeviceBuffer weights, partial, raw, coef, hpart, hsum, model_stage, out_stage, misfit_stage,
-      grad_stage, farpart, nearpart, coef32, coef_mono, near_h, near_v, vsites, partsum,
+  jgm::DeviceBuffer weights, partial, raw, coef, hpart, hsum, out_stage, misfit_stage,
+      farpart, nearpart, coef32, coef_mono, near_h, near_v, vsites, partsum,
       chunk_scratch, mag_part;
+  // operands of the host-pointer entry points (small calls): device buffers, and the
+  // page-locked memory their copies pass through
+  jgm::DeviceBuffer host_stage[3];
+  void* host_pin = nullptr;
   // FP64 evaluation of the sites the mixed path hands back (corner weights, partials,
   // sums, gathered misfits, coefficients, corner sums, a gradient, the residuals of the
   // other sites)
