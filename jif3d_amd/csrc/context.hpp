@@ -106,6 +106,16 @@ struct SlabMesh {
   DeviceBuffer rho, sums, rmt, gv, rm0;
 };
 
+// FP64 far field by tile expansions (tile_far.hip), for the gz kind (index 0) and gz + FTG (1):
+// whether the geometry of generation gen takes it, the harmonic polynomials' tables (made
+// once), the tiles' centres (of geo_gen), and per call the tiles' coefficients, corner weights,
+// reference density and local coefficients.
+struct TileFar {
+  unsigned long gen[2] = {0, 0}, geo_gen = 0;
+  bool chosen[2] = {false, false}, tables = false;
+  DeviceBuffer ptr, idx, cptr, cidx, mono, val, cval, geo, coefs, wt, ref, lam;
+};
+
 // Optional per-kernel timing: HIP events recorded on the context's stream around
 // each launch, harvested lazily.
 struct Profiler {
@@ -211,6 +221,7 @@ struct jgm_context {
   jgm::DeviceBuffer bgT;  // [S][L][7] background box terms, valid when bg_valid
   bool bg_valid = false;
   jgm::NearBoxes near;
+  jgm::TileFar tile_far;
 
   // scratch
   jgm::DeviceBuffer weights, partial, raw, coef, hpart, hsum, out_stage, misfit_stage,
@@ -281,6 +292,13 @@ hipError_t launch_forward_fp64_batch(jgm_context* ctx, int kind, size_t nmodels,
 hipError_t launch_adjoint_fp64_batch(jgm_context* ctx, int kind, size_t nsets,
                                      const double* raw_misfits, size_t misfit_ld, double* grads,
                                      size_t grad_ld);
+// tile expansions: whether the kind takes them on this geometry (tables and centres made);
+// the corner sums of one model as nchunks rows of partial[chunk][component][site]; the cells'
+// gradient of per-site corner-sum coefficients coef[site][component]
+hipError_t tile_far_prepare(jgm_context* ctx, int kind, bool* applies);
+hipError_t tile_far_forward(jgm_context* ctx, int kind, const double* model, double** partial,
+                            int* nchunks);
+hipError_t tile_far_adjoint(jgm_context* ctx, int kind, const double* coef, double* grad);
 hipError_t launch_misfit_to_raw(jgm_context* ctx, int kind, const double* misfit,
                                 const double* raw, double* raw_misfit);
 hipError_t launch_sensitivity_rows(jgm_context* ctx, int kind, size_t site0, size_t nsites,

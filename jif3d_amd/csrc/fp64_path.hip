@@ -1,4 +1,5 @@
-// FP64 closed-form path: corner-first forward and adjoint, 1-D background,
+// FP64 path: corner-first closed form forward and adjoint (large meshes of the gz and gz + FTG
+// kinds through the tile expansions of tile_far.hip), 1-D background,
 // epilogues (component assembly, magnetic projection, data transforms) and the
 // per-cell sensitivity rows.
 //
@@ -691,6 +692,41 @@ hipError_t adjoint_impl(jgm_context* ctx, int kind, int nb, const double* rm, si
     }
   }
   return hipGetLastError();
+}
+
+// One model's data, one residual set's gradient through the tile expansions.
+template <int MASK>
+hipError_t forward_tiles(jgm_context* ctx, int kind, const double* model, double* out,
+                         double* raw_out) {
+  constexpr int NC = Ncomp<MASK>::value;
+  const int S = (int)ctx->S;
+  double* part = nullptr;
+  int nchunks = 0;
+  hipError_t e = tile_far_forward(ctx, kind, model, &part, &nchunks);
+  if (e != hipSuccess) return e;
+  if ((e = ctx->partsum.ensure(sizeof(double) * (size_t)NC * S)) != hipSuccess) return e;
+  if ((e = launch_reduce_chunks(ctx, part, nchunks, (long)NC * S, ctx->partsum.as<double>())) !=
+      hipSuccess)
+    return e;
+  hipLaunchKernelGGL((k_forward_finish<MASK>), dim3(blocks_for(S)), dim3(kBlock), 0, ctx->stream,
+                     ctx->partsum.as<const double>(), 1, S, ctx->bgT.as<const double>(),
+                     model + ncells(ctx), (int)ctx->bgthick.size(), kind, field_dir(ctx),
+                     ctx->transform, std::cos(ctx->tf_inc) * std::cos(ctx->tf_dec),
+                     std::cos(ctx->tf_inc) * std::sin(ctx->tf_dec), std::sin(ctx->tf_inc), out,
+                     raw_out);
+  return hipGetLastError();
+}
+
+template <int MASK>
+hipError_t adjoint_tiles(jgm_context* ctx, int kind, const double* rm, double* grad) {
+  constexpr int NC = Ncomp<MASK>::value;
+  const int S = (int)ctx->S;
+  hipError_t e = ctx->coef.ensure(sizeof(double) * (size_t)S * NC);
+  if (e != hipSuccess) return e;
+  hipLaunchKernelGGL((k_adjoint_coef<MASK>), dim3(blocks_for(S)), dim3(kBlock), 0, ctx->stream, rm,
+                     S, kind, field_dir(ctx), ctx->coef.as<double>(), NC);
+  if ((e = tile_far_adjoint(ctx, kind, ctx->coef.as<const double>(), grad)) != hipSuccess) return e;
+  return launch_background_gradient(ctx, kind, rm, grad + ncells(ctx));
 }
 
 // ---------------------------------------------------------------------------
@@ -1523,6 +1559,19 @@ hipError_t launch_forward_fp64(jgm_context* ctx, int kind, const double* model, 
 hipError_t launch_forward_fp64_batch(jgm_context* ctx, int kind, size_t nmodels,
                                      const double* models, size_t model_ld, double* out,
                                      size_t out_ld, double* raw_out, size_t raw_ld) {
+  bool tiles = false;
+  if (hipError_t e = tile_far_prepare(ctx, kind, &tiles); e != hipSuccess) return e;
+  if (tiles) {
+    for (size_t b = 0; b < nmodels; ++b) {
+      const double* m = models + b * model_ld;
+      double* o = out + b * out_ld;
+      double* r = raw_out ? raw_out + b * raw_ld : nullptr;
+      const hipError_t e = kind == JGM_KIND_SCALAR ? forward_tiles<kMaskScalar>(ctx, kind, m, o, r)
+                                                   : forward_tiles<kMaskAll>(ctx, kind, m, o, r);
+      if (e != hipSuccess) return e;
+    }
+    return hipSuccess;
+  }
   for (size_t b0 = 0; b0 < nmodels;) {
     const size_t left = nmodels - b0;
     const int nb = left >= 8 ? 8 : left >= 4 ? 4 : left >= 2 ? 2 : 1;
@@ -1572,6 +1621,18 @@ hipError_t launch_adjoint_fp64(jgm_context* ctx, int kind, const double* /*model
 hipError_t launch_adjoint_fp64_batch(jgm_context* ctx, int kind, size_t nsets,
                                      const double* raw_misfits, size_t misfit_ld, double* grads,
                                      size_t grad_ld) {
+  bool tiles = false;
+  if (hipError_t e = tile_far_prepare(ctx, kind, &tiles); e != hipSuccess) return e;
+  if (tiles) {
+    for (size_t b = 0; b < nsets; ++b) {
+      const double* r = raw_misfits + b * misfit_ld;
+      double* g = grads + b * grad_ld;
+      const hipError_t e = kind == JGM_KIND_SCALAR ? adjoint_tiles<kMaskScalar>(ctx, kind, r, g)
+                                                   : adjoint_tiles<kMaskAll>(ctx, kind, r, g);
+      if (e != hipSuccess) return e;
+    }
+    return hipSuccess;
+  }
   for (size_t b0 = 0; b0 < nsets;) {
     const size_t left = nsets - b0;
     const int nb = left >= 8 ? 8 : left >= 4 ? 4 : left >= 2 ? 2 : 1;
