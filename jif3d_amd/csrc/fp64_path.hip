@@ -440,14 +440,31 @@ __global__ __launch_bounds__(kBlock) void k_sensitivity_rows(
 }
 
 // Sensitivity rows on a mesh whose cells share their corners: a workgroup evaluates the corner
-// terms of a brick of kTileI x kTileJ corner columns for one site into LDS once and forms the
-// box sums of its cells from there, in box_terms_f64's order of additions, so each entry
-// sums what eight corners of its own would give it.  A brick of 5 x 6 columns and up to 34
-// corners each costs 1.6 corner evaluations per cell instead of 8; 512 threads and at most
-// 63 KB of LDS put two workgroups on a CU.  For the vertical gradient a corner carries the z
-// column at the site and 1 m below.  FTG rows of 64 sites over 64 x 64 x 32 cells: 0.61 ms with
-// eight evaluations per cell, 0.21 ms here; the 604 MB written take 0.12 ms at a copy's rate.
+// terms of a brick of cells for one site into LDS and forms the cells' box sums from there, in
+// box_terms_f64's order of additions.  Up to 33 cells deep; two forms:
+//  * gz and gz + FTG: a brick of 4 x 5 columns, each mesh corner once (1.6 evaluations per cell
+//    instead of 8).
+//  * the tensor alone and the vertical gradient (which carries the z column at the site and 1 m
+//    below): 7 columns along y, each with its own four corner edges, shared down the column (4.1
+//    per cell).  Down a line of corners that passes near the site log(u + r) turns an ulp of r
+//    into up to 1e-7 of a row's rms, and these rows have no larger component to hide it: the four
+//    edges of a column round r^2 each in its own way (edge_r2), as a cell by itself does, and the
+//    entries keep that rounding.
+// 512 threads and at most 63 KB of LDS put two workgroups on a CU.  Rows of 64 sites over
+// 64 x 64 x 32 cells: gz + FTG @@ ms (eight evaluations per cell @@), FTG @@ ms (0.61); the
+// 604 MB of the FTG rows take 0.12 ms at a copy's rate.
 constexpr int kTileI = 5, kTileJ = 6, kTileK = 34, kTileThreads = 512;
+constexpr int kColumns = 7;
+
+// r^2 from the offsets to edge (a, b) of a cell: the products that a cell's eight corners share
+// are rounded, the others fused.
+__device__ __forceinline__ double edge_r2(int a, int b, double x, double y, double z) {
+#pragma clang fp contract(off)
+  const double xx = x * x, yy = y * y, zz = z * z;
+  if (a == 0 && b == 0) return fma(z, z, fma(x, x, yy));
+  const double s = b == 0 ? fma(x, x, yy) : a == 0 ? fma(y, y, xx) : xx + yy;
+  return s + zz;
+}
 
 template <int MASK, bool TWO>
 __global__ __launch_bounds__(kTileThreads) void k_sensitivity_row_tiles(
@@ -458,7 +475,10 @@ __global__ __launch_bounds__(kTileThreads) void k_sensitivity_row_tiles(
     double* __restrict__ rows) {
   constexpr int NC = Ncomp<MASK>::value;
   constexpr int NV = TWO ? 2 * NC : NC;
-  __shared__ double val[NV][kTileI * kTileJ * kTileK];
+  constexpr bool EDGES = (MASK & kGz) == 0;  // columns with edges of their own
+  constexpr int TI = EDGES ? 1 : kTileI - 1, TJ = EDGES ? kColumns : kTileJ - 1;
+  constexpr int NCORNER = EDGES ? 4 * kColumns * kTileK : kTileI * kTileJ * kTileK;
+  __shared__ double val[NV][NCORNER];
   __shared__ LogTableShared tab;
   const LogTable lg = tab.fill();
   const long N = (long)nx * ny * nz;
@@ -467,21 +487,26 @@ __global__ __launch_bounds__(kTileThreads) void k_sensitivity_row_tiles(
   const int kraw = (int)raw_per_site(kind);
   double* site_rows = rows + (long)blockIdx.y * kraw * np;
   const int tk = (int)blockIdx.x % tiles_k, tij = (int)blockIdx.x / tiles_k;
-  const int i0 = tij / tiles_j * (kTileI - 1), j0 = tij % tiles_j * (kTileJ - 1), k0 = tk * cells_k;
-  const int ni = min(kTileI - 1, nx - i0), nj = min(kTileJ - 1, ny - j0), nk = min(cells_k, nz - k0);
+  const int i0 = tij / tiles_j * TI, j0 = tij % tiles_j * TJ, k0 = tk * cells_k;
+  const int ni = min(TI, nx - i0), nj = min(TJ, ny - j0), nk = min(cells_k, nz - k0);
   const double px = sx[s], py = sy[s], pz = sz[s];
-  const int ck = nk + 1, ncorner = (ni + 1) * (nj + 1) * ck;
+  const int ck = nk + 1, ncorner = (EDGES ? 4 * nj : (ni + 1) * (nj + 1)) * ck;
   for (int q = threadIdx.x; q < ncorner; q += kTileThreads) {
-    const int k = q % ck, ij = q / ck, j = ij % (nj + 1), i = ij / (nj + 1);
+    const int k = q % ck, e = q / ck;
+    // edge (a, b) of column j, or corner column (i, j)
+    const int a = EDGES ? e & 1 : 0, b = EDGES ? (e >> 1) & 1 : 0;
+    const int i = EDGES ? a : e / (nj + 1), j = EDGES ? (e >> 2) + b : e % (nj + 1);
     const double x = px - Xc[i0 + i], y = py - Yc[j0 + j];
-    double t[NC];
-    corner_terms_f64<MASK>(x, y, pz - Zc[k0 + k], t, lg);
 #pragma unroll
-    for (int m = 0; m < NC; ++m) val[m][q] = t[m];
-    if constexpr (TWO) {
-      corner_terms_f64<MASK>(x, y, (pz + 1.0) - Zc[k0 + k], t, lg);
+    for (int h = 0; h < (TWO ? 2 : 1); ++h) {
+      const double z = (h == 0 ? pz : pz + 1.0) - Zc[k0 + k];
+      double t[NC];
+      if constexpr (EDGES)
+        corner_terms_r2_f64<MASK>(x, y, z, edge_r2(a, b, x, y, z), t, lg);
+      else
+        corner_terms_f64<MASK>(x, y, z, t, lg);
 #pragma unroll
-      for (int m = 0; m < NC; ++m) val[NC + m][q] = t[m];
+      for (int m = 0; m < NC; ++m) val[h * NC + m][q] = t[m];
     }
   }
   __syncthreads();
@@ -490,8 +515,8 @@ __global__ __launch_bounds__(kTileThreads) void k_sensitivity_row_tiles(
   const int ncell = ni * nj * nk;
   for (int c = threadIdx.x; c < ncell; c += kTileThreads) {
     const int k = c % nk, ij = c / nk, j = ij % nj, i = ij / nj;
-    const int q = (i * (nj + 1) + j) * ck + k;
-    const int di = (nj + 1) * ck, dj = ck;
+    const int q = (EDGES ? 4 * j : i * (nj + 1) + j) * ck + k;
+    const int di = (EDGES ? 1 : nj + 1) * ck, dj = (EDGES ? 2 : 1) * ck;
     double v[NV];
 #pragma unroll
     for (int m = 0; m < NV; ++m) {
@@ -1672,8 +1697,9 @@ hipError_t launch_sensitivity_rows(jgm_context* ctx, int kind, size_t site0, siz
                             : ctx->fieldstrength * (1e-7 / kGravConst);
   const size_t n[3] = {ctx->nx, ctx->ny, ctx->nz};
   if (ctx->shared_corners && ncells(ctx) > 0) {
-    const int tiles_i = (int)((n[0] + kTileI - 2) / (kTileI - 1));
-    const int tiles_j = (int)((n[1] + kTileJ - 2) / (kTileJ - 1));
+    const bool edges = mask_of(kind) == kMaskTensor;
+    const size_t ti = edges ? 1 : kTileI - 1, tj = edges ? kColumns : kTileJ - 1;
+    const int tiles_i = (int)((n[0] + ti - 1) / ti), tiles_j = (int)((n[1] + tj - 1) / tj);
     const int tiles_k = (int)((n[2] + kTileK - 2) / (kTileK - 1));
     const int cells_k = (int)((n[2] + tiles_k - 1) / tiles_k);
     const long tiles = (long)tiles_i * tiles_j * tiles_k;

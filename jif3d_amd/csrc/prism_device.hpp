@@ -234,9 +234,8 @@ __device__ __forceinline__ void diag_terms_f64(double x, double y, double z, dou
 }
 
 template <int MASK, class Log = LogPoly>
-__device__ __forceinline__ void corner_terms_f64(double x, double y, double z, double* t,
-                                                 Log lg = {}) {
-  const double r2 = x * x + y * y + z * z;
+__device__ __forceinline__ void corner_terms_r2_f64(double x, double y, double z, double r2,
+                                                    double* t, Log lg = {}) {
   if constexpr (MASK == kMaskZcol) {
     const double r = sqrt(r2);
     // Uzz = atan2(x y, z r), Uxz = log(max(y + r, eps)), Uyz = log(max(x + r, eps)); the
@@ -321,6 +320,12 @@ __device__ __forceinline__ void corner_terms_f64(double x, double y, double z, d
       t[k++] = atan2(x * y, z * r);
     }
   }
+}
+
+template <int MASK, class Log = LogPoly>
+__device__ __forceinline__ void corner_terms_f64(double x, double y, double z, double* t,
+                                                 Log lg = {}) {
+  corner_terms_r2_f64<MASK>(x, y, z, x * x + y * y + z * z, t, lg);
 }
 
 // Sign and scale applied to each accumulated corner sum, in the kernel's

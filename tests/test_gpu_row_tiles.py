@@ -1,5 +1,5 @@
 """Sensitivity rows evaluated corner by corner in bricks of the mesh, at mesh sizes around the
-brick's edges (4 x 5 columns of at most 33 cells), for every kind against the oracle's rows, and
+bricks' edges (4 x 5 or 1 x 7 columns of at most 33 cells), for every kind against the oracle's rows, and
 on a mesh whose cells do not share their corners (a gap beside a layer of cells), where every
 cell takes its own eight corners and the other cells' entries stay the same.  Bounds of the FP64 path: 1e-12 of the largest entry for gz, 1e-11
 for the tensor and magnetic kinds, plus, entry by entry, the rounding of the closed form itself:
@@ -17,7 +17,7 @@ from jif3d_amd.model import (ThreeDGravityModel, ThreeDSusceptibilityModel,
 
 pytestmark = pytest.mark.gpu
 FIELD = (0.9, 0.2, 48000.0)
-MESHES = [(1, 1, 1), (4, 5, 33), (5, 6, 34), (9, 11, 1), (3, 2, 67), (8, 5, 66)]
+MESHES = [(1, 1, 1), (4, 5, 33), (5, 6, 34), (9, 11, 1), (3, 2, 67), (8, 5, 66), (2, 7, 33), (3, 15, 35)]
 
 
 def geometry(kind, dims, nsites=3):
