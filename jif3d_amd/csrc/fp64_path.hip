@@ -64,7 +64,9 @@ __global__ __launch_bounds__(kBlock) void k_corner_weights(const double* __restr
 // Forward: one lane per site; the wave walks a chunk of corner columns (I, J)
 // and all K.  Corner coordinates and weights are wave-uniform (scalar loads).  NB
 // models share every corner evaluation (weights w[q * NB + b]); the partial sums of
-// model b go to partial[((b * nchunks + chunk) * NC + m) * S + s].
+// model b go to partial[((b * nchunks + chunk) * NC + m) * S + s].  A workgroup's waves past the
+// last site end at once, and the chunks are counted by the waves that stay (64 sites, 96 x 96 x 64
+// cells, gz + FTG: 0.42 ms, 1.08 ms when all four waves walked).
 template <int MASK, int NB>
 __global__ __launch_bounds__(kBlock) void k_forward_corners(
     const double* __restrict__ sx, const double* __restrict__ sy, const double* __restrict__ sz,
@@ -75,6 +77,7 @@ __global__ __launch_bounds__(kBlock) void k_forward_corners(
   __shared__ LogTableShared tab;
   const LogTable lg = tab.fill();
   const int s = blockIdx.x * blockDim.x + threadIdx.x;
+  if (s - (int)(threadIdx.x & 63) >= S) return;
   const int sl = s < S ? s : S - 1;
   const double px = sx[sl], py = sy[sl], pz = sz[sl];
   const long col0 = (long)blockIdx.y * cols_per_chunk;
@@ -451,7 +454,7 @@ __global__ __launch_bounds__(kBlock) void k_sensitivity_rows(
 //    edges of a column round r^2 each in its own way (edge_r2), as a cell by itself does, and the
 //    entries keep that rounding.
 // 512 threads and at most 63 KB of LDS put two workgroups on a CU.  Rows of 64 sites over
-// 64 x 64 x 32 cells: gz + FTG @@ ms (eight evaluations per cell @@), FTG @@ ms (0.61); the
+// 64 x 64 x 32 cells: gz + FTG 0.26 ms (eight evaluations per cell 0.68), FTG 0.40 ms (0.61); the
 // 604 MB of the FTG rows take 0.12 ms at a copy's rate.
 constexpr int kTileI = 5, kTileJ = 6, kTileK = 34, kTileThreads = 512;
 constexpr int kColumns = 7;
@@ -612,7 +615,7 @@ hipError_t forward_impl(jgm_context* ctx, int kind, int nb, const double* models
   const int site_blocks = (S + kBlock - 1) / kBlock;
   int nchunks = 1;
   if (N > 0) {
-    const long waves_per_chunk = (long)site_blocks * (kBlock / 64);
+    const long waves_per_chunk = (S + 63) / 64;
     long want = (kTargetWaves + waves_per_chunk - 1) / waves_per_chunk;
     want = std::min<long>(want, ncols);
     nchunks = (int)std::max<long>(1, want);
@@ -840,6 +843,7 @@ __global__ __launch_bounds__(kBlock) void k_forward_corners_mag3(
   __shared__ LogTableShared tab;
   const LogTable lg = tab.fill();
   const int s = blockIdx.x * blockDim.x + threadIdx.x;
+  if (s - (int)(threadIdx.x & 63) >= S) return;
   const int sl = s < S ? s : S - 1;
   const double px = sx[sl], py = sy[sl], pz = sz[sl];
   const long col0 = (long)blockIdx.y * cols_per_chunk;
@@ -922,8 +926,7 @@ __global__ __launch_bounds__(kBlock) void k_mag3_coef(const double* __restrict__
 
 // chunking of a lane-per-site corner walk (as forward_impl)
 void site_chunks(long S, long ncols, long* nchunks, long* cols_per_chunk) {
-  const long site_blocks = (S + kBlock - 1) / kBlock;
-  const long waves_per_chunk = site_blocks * (kBlock / 64);
+  const long waves_per_chunk = (S + 63) / 64;
   long want = (kTargetWaves + waves_per_chunk - 1) / waves_per_chunk;
   want = std::max<long>(1, std::min<long>(want, ncols));
   *cols_per_chunk = (ncols + want - 1) / want;
@@ -1234,7 +1237,7 @@ hipError_t forward_sites_impl(jgm_context* ctx, int kind, const double* model, i
   const int ncx = (int)ctx->nx + 1, ncy = (int)ctx->ny + 1, ncz = (int)ctx->nz + 1;
   const long ncols = (long)ncx * ncy;
   const int site_blocks = (F + kBlock - 1) / kBlock;
-  const long waves_per_chunk = (long)site_blocks * (kBlock / 64);
+  const long waves_per_chunk = (F + 63) / 64;
   long want = std::min<long>((kTargetWaves + waves_per_chunk - 1) / waves_per_chunk, ncols);
   want = std::max<long>(1, want);
   const long per = (ncols + want - 1) / want;
@@ -1457,7 +1460,7 @@ hipError_t forward_noalloc_impl(jgm_context* ctx, int kind, double* base, const 
   NoallocPlan plan;
   int nchunks = 0;
   if (N > 0) {
-    const long waves_per_chunk = (long)site_blocks * (kBlock / 64);
+    const long waves_per_chunk = (S + 63) / 64;
     long want = std::min<long>((kTargetWaves + waves_per_chunk - 1) / waves_per_chunk, ncols);
     want = std::max<long>(1, want);
     while (want > 1 && noalloc_layout(&plan, L, S, nq, NC, (int)want) > kNoallocDoubles)

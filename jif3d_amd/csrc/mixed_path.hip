@@ -547,6 +547,7 @@ __attribute__((amdgpu_waves_per_eu(far_fwd_waves(NB, MESH, MASK)))) void k_far_f
     long tiles_per_chunk, double* __restrict__ farpart) {
   constexpr int NC = Ncomp<MASK>::value;
   const int li = blockIdx.x * blockDim.x + threadIdx.x;
+  if (li - (int)(threadIdx.x & 63) >= S) return;  // the wave has no site
   const int s = order[li < S ? li : S - 1];
   const double px = sx[s], py = sy[s], pz = sz[s];
   int bx[6];
@@ -1414,7 +1415,7 @@ hipError_t forward_mixed_impl(jgm_context* ctx, int kind, int nbm, const double*
   if ((e = ctx->nearpart.ensure(sizeof(double) * (size_t)nbm * S * NC)) != hipSuccess) return e;
   if (N > 0) {
     const int site_blocks = (S + kBlock - 1) / kBlock;
-    const long waves_per_chunk = (long)site_blocks * (kBlock / 64);
+    const long waves_per_chunk = (S + 63) / 64;
     long want = (ctx->far_fwd_waves + waves_per_chunk - 1) / waves_per_chunk;
     want = std::max<long>(1, std::min<long>(want, ntiles));
     const long per = (ntiles + want - 1) / want;

@@ -134,6 +134,7 @@ __global__ __launch_bounds__(kBlock) void k_storedj_build(
   // functions) rather than the table of the corner kernels
   const std::conditional_t<MASK == kMaskScalar, LogLibrary, LogPoly> lg;
   const int s = blockIdx.x * blockDim.x + threadIdx.x;
+  if (s - (int)(threadIdx.x & 63) >= S) return;  // the wave has no site
   const int sl = s < S ? s : S - 1;
   const double px = sx[sl], py = sy[sl], pz = sz[sl];
   const int kJ = compact_rows(kind);
@@ -1075,7 +1076,7 @@ hipError_t build_columns(jgm_context* ctx, int kind, long c0, long c1, long ld, 
   const int S = (int)ctx->S;
   const int site_blocks = (S + kBlock - 1) / kBlock;
   const long n = c1 - c0;
-  const long waves_per_chunk = (long)site_blocks * (kBlock / 64);
+  const long waves_per_chunk = (S + 63) / 64;
   long want = std::max<long>(1, std::min<long>(n, (16384 + waves_per_chunk - 1) / waves_per_chunk));
   const int ny = (int)ctx->ny, nz = (int)ctx->nz;
   long per = (n + want - 1) / want;
