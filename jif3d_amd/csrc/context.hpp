@@ -293,12 +293,15 @@ hipError_t launch_adjoint_fp64_batch(jgm_context* ctx, int kind, size_t nsets,
                                      const double* raw_misfits, size_t misfit_ld, double* grads,
                                      size_t grad_ld);
 // tile expansions: whether the kind takes them on this geometry (tables and centres made);
-// the corner sums of one model as nchunks rows of partial[chunk][component][site]; the cells'
-// gradient of per-site corner-sum coefficients coef[site][component]
+// how many of the models left a launch takes (8, 4, 2 or 1); their corner sums as nchunks rows each
+// of partial[model][chunk][component][site]; the cells' gradients of per-site corner-sum
+// coefficients coef[set][site][component]
 hipError_t tile_far_prepare(jgm_context* ctx, int kind, bool* applies);
-hipError_t tile_far_forward(jgm_context* ctx, int kind, const double* model, double** partial,
-                            int* nchunks);
-hipError_t tile_far_adjoint(jgm_context* ctx, int kind, const double* coef, double* grad);
+int tile_far_models(const jgm_context* ctx, int kind, size_t left);
+hipError_t tile_far_forward(jgm_context* ctx, int kind, int nb, const double* models,
+                            size_t model_ld, double** partial, int* nchunks);
+hipError_t tile_far_adjoint(jgm_context* ctx, int kind, int nb, const double* coef, double* grads,
+                            size_t grad_ld);
 hipError_t launch_misfit_to_raw(jgm_context* ctx, int kind, const double* misfit,
                                 const double* raw, double* raw_misfit);
 hipError_t launch_sensitivity_rows(jgm_context* ctx, int kind, size_t site0, size_t nsites,

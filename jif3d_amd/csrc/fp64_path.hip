@@ -722,39 +722,52 @@ hipError_t adjoint_impl(jgm_context* ctx, int kind, int nb, const double* rm, si
   return hipGetLastError();
 }
 
-// One model's data, one residual set's gradient through the tile expansions.
+// Data of nb models, gradients of nb residual sets through the tile expansions; nb as above.
 template <int MASK>
-hipError_t forward_tiles(jgm_context* ctx, int kind, const double* model, double* out,
-                         double* raw_out) {
+hipError_t forward_tiles(jgm_context* ctx, int kind, int nb, const double* models, size_t model_ld,
+                         double* out, size_t out_ld, double* raw_out, size_t raw_ld) {
   constexpr int NC = Ncomp<MASK>::value;
   const int S = (int)ctx->S;
   double* part = nullptr;
   int nchunks = 0;
-  hipError_t e = tile_far_forward(ctx, kind, model, &part, &nchunks);
+  hipError_t e = tile_far_forward(ctx, kind, nb, models, model_ld, &part, &nchunks);
   if (e != hipSuccess) return e;
-  if ((e = ctx->partsum.ensure(sizeof(double) * (size_t)NC * S)) != hipSuccess) return e;
-  if ((e = launch_reduce_chunks(ctx, part, nchunks, (long)NC * S, ctx->partsum.as<double>())) !=
-      hipSuccess)
-    return e;
-  hipLaunchKernelGGL((k_forward_finish<MASK>), dim3(blocks_for(S)), dim3(kBlock), 0, ctx->stream,
-                     ctx->partsum.as<const double>(), 1, S, ctx->bgT.as<const double>(),
-                     model + ncells(ctx), (int)ctx->bgthick.size(), kind, field_dir(ctx),
-                     ctx->transform, std::cos(ctx->tf_inc) * std::cos(ctx->tf_dec),
-                     std::cos(ctx->tf_inc) * std::sin(ctx->tf_dec), std::sin(ctx->tf_inc), out,
-                     raw_out);
+  const long n = (long)NC * S;
+  if ((e = ctx->partsum.ensure(sizeof(double) * (size_t)n)) != hipSuccess) return e;
+  for (int b = 0; b < nb; ++b) {
+    if ((e = launch_reduce_chunks(ctx, part + b * nchunks * n, nchunks, n,
+                                  ctx->partsum.as<double>())) != hipSuccess)
+      return e;
+    hipLaunchKernelGGL((k_forward_finish<MASK>), dim3(blocks_for(S)), dim3(kBlock), 0, ctx->stream,
+                       ctx->partsum.as<const double>(), 1, S, ctx->bgT.as<const double>(),
+                       models + b * model_ld + ncells(ctx), (int)ctx->bgthick.size(), kind,
+                       field_dir(ctx), ctx->transform,
+                       std::cos(ctx->tf_inc) * std::cos(ctx->tf_dec),
+                       std::cos(ctx->tf_inc) * std::sin(ctx->tf_dec), std::sin(ctx->tf_inc),
+                       out + b * out_ld, raw_out ? raw_out + b * raw_ld : nullptr);
+  }
   return hipGetLastError();
 }
 
 template <int MASK>
-hipError_t adjoint_tiles(jgm_context* ctx, int kind, const double* rm, double* grad) {
+hipError_t adjoint_tiles(jgm_context* ctx, int kind, int nb, const double* rm, size_t rm_ld,
+                         double* grads, size_t grad_ld) {
   constexpr int NC = Ncomp<MASK>::value;
   const int S = (int)ctx->S;
-  hipError_t e = ctx->coef.ensure(sizeof(double) * (size_t)S * NC);
+  hipError_t e = ctx->coef.ensure(sizeof(double) * (size_t)nb * S * NC);
   if (e != hipSuccess) return e;
-  hipLaunchKernelGGL((k_adjoint_coef<MASK>), dim3(blocks_for(S)), dim3(kBlock), 0, ctx->stream, rm,
-                     S, kind, field_dir(ctx), ctx->coef.as<double>(), NC);
-  if ((e = tile_far_adjoint(ctx, kind, ctx->coef.as<const double>(), grad)) != hipSuccess) return e;
-  return launch_background_gradient(ctx, kind, rm, grad + ncells(ctx));
+  for (int b = 0; b < nb; ++b)
+    hipLaunchKernelGGL((k_adjoint_coef<MASK>), dim3(blocks_for(S)), dim3(kBlock), 0, ctx->stream,
+                       rm + b * rm_ld, S, kind, field_dir(ctx),
+                       ctx->coef.as<double>() + (size_t)b * S * NC, NC);
+  if ((e = tile_far_adjoint(ctx, kind, nb, ctx->coef.as<const double>(), grads, grad_ld)) !=
+      hipSuccess)
+    return e;
+  for (int b = 0; b < nb; ++b)
+    if ((e = launch_background_gradient(ctx, kind, rm + b * rm_ld,
+                                        grads + b * grad_ld + ncells(ctx))) != hipSuccess)
+      return e;
+  return hipSuccess;
 }
 
 // ---------------------------------------------------------------------------
@@ -1590,13 +1603,17 @@ hipError_t launch_forward_fp64_batch(jgm_context* ctx, int kind, size_t nmodels,
   bool tiles = false;
   if (hipError_t e = tile_far_prepare(ctx, kind, &tiles); e != hipSuccess) return e;
   if (tiles) {
-    for (size_t b = 0; b < nmodels; ++b) {
+    for (size_t b = 0; b < nmodels;) {
+      const int nb = tile_far_models(ctx, kind, nmodels - b);
       const double* m = models + b * model_ld;
       double* o = out + b * out_ld;
       double* r = raw_out ? raw_out + b * raw_ld : nullptr;
-      const hipError_t e = kind == JGM_KIND_SCALAR ? forward_tiles<kMaskScalar>(ctx, kind, m, o, r)
-                                                   : forward_tiles<kMaskAll>(ctx, kind, m, o, r);
+      const hipError_t e =
+          kind == JGM_KIND_SCALAR
+              ? forward_tiles<kMaskScalar>(ctx, kind, nb, m, model_ld, o, out_ld, r, raw_ld)
+              : forward_tiles<kMaskAll>(ctx, kind, nb, m, model_ld, o, out_ld, r, raw_ld);
       if (e != hipSuccess) return e;
+      b += nb;
     }
     return hipSuccess;
   }
@@ -1652,12 +1669,16 @@ hipError_t launch_adjoint_fp64_batch(jgm_context* ctx, int kind, size_t nsets,
   bool tiles = false;
   if (hipError_t e = tile_far_prepare(ctx, kind, &tiles); e != hipSuccess) return e;
   if (tiles) {
-    for (size_t b = 0; b < nsets; ++b) {
+    for (size_t b = 0; b < nsets;) {
+      const int nb = tile_far_models(ctx, kind, nsets - b);
       const double* r = raw_misfits + b * misfit_ld;
       double* g = grads + b * grad_ld;
-      const hipError_t e = kind == JGM_KIND_SCALAR ? adjoint_tiles<kMaskScalar>(ctx, kind, r, g)
-                                                   : adjoint_tiles<kMaskAll>(ctx, kind, r, g);
+      const hipError_t e =
+          kind == JGM_KIND_SCALAR
+              ? adjoint_tiles<kMaskScalar>(ctx, kind, nb, r, misfit_ld, g, grad_ld)
+              : adjoint_tiles<kMaskAll>(ctx, kind, nb, r, misfit_ld, g, grad_ld);
       if (e != hipSuccess) return e;
+      b += nb;
     }
     return hipSuccess;
   }

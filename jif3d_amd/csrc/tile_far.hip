@@ -26,6 +26,7 @@
 #include <algorithm>
 #include <cmath>
 #include <complex>
+#include <type_traits>
 #include <vector>
 
 #include "context.hpp"
@@ -97,7 +98,7 @@ __device__ __forceinline__ Tile tile_of(const TileGrid& g, int t) {
 // Workgroup b of the kernels that take a tile each: layer by layer from the top.  Workgroups go
 // to the eight XCDs in turn, and in the tiles' own order (z fastest) a mesh of eight layers of
 // tiles gives each XCD one layer, the uppermost with nearly all near sites (near gradient of
-// 2048 tiles and 4096 sites 5.8 ms, @@ ms this way).
+// 2048 tiles and 4096 sites 5.8 ms, 2.0 ms this way).
 __device__ __forceinline__ int tile_of_block(const TileGrid& g, int b) {
   const int columns = g.tx * g.ty;
   return b % columns * g.tz + b / columns;
@@ -130,23 +131,26 @@ __device__ __forceinline__ Offset offset_of(double px, double py, double pz, dou
 // Mean of 1024 cells spread over the mesh.  The tiles carry the densities less this value and
 // the whole mesh as one box carries it: what a nearly uniform model's cells have in common
 // cancels before any truncation, as it does in the corner weights of the closed form.
-__global__ __launch_bounds__(1024) void k_reference_density(const double* __restrict__ rho, long n,
+__global__ __launch_bounds__(1024) void k_reference_density(const double* __restrict__ rho,
+                                                            long ld, long n,
                                                             double* __restrict__ ref) {
   __shared__ double red[1024];
+  rho += blockIdx.x * ld;
   red[threadIdx.x] = rho[(long)((2.0 * threadIdx.x + 1.0) * (double)n / 2048.0)];
   __syncthreads();
   for (int w = 512; w > 0; w >>= 1) {
     if ((int)threadIdx.x < w) red[threadIdx.x] += red[threadIdx.x + w];
     __syncthreads();
   }
-  if (threadIdx.x == 0) ref[0] = red[0] * (1.0 / 1024.0);
+  if (threadIdx.x == 0) ref[blockIdx.x] = red[0] * (1.0 / 1024.0);
 }
 
-// Corner sums of the mesh as one box of the reference density: one row of partial.
+// Corner sums of the mesh as one box of the reference density: one row of partial a model.
 template <int MASK>
 __global__ __launch_bounds__(kBlock) void k_reference_box(
     const double* __restrict__ sx, const double* __restrict__ sy, const double* __restrict__ sz,
-    int S, TileGrid g, const double* __restrict__ ref, double* __restrict__ partial) {
+    int S, TileGrid g, const double* __restrict__ ref, int nb, double* __restrict__ partial,
+    long ld) {
   constexpr int NC = Ncomp<MASK>::value;
   __shared__ LogTableShared tab;
   const LogTable lg = tab.fill();
@@ -163,8 +167,9 @@ __global__ __launch_bounds__(kBlock) void k_reference_box(
 #pragma unroll
     for (int m = 0; m < NC; ++m) acc[m] += plus ? v[m] : -v[m];
   }
+  for (int b = 0; b < nb; ++b)
 #pragma unroll
-  for (int m = 0; m < NC; ++m) partial[(long)m * S + s] = acc[m] * ref[0];
+    for (int m = 0; m < NC; ++m) partial[b * ld + (long)m * S + s] = acc[m] * ref[b];
 }
 
 // Integrals over the tile's cells of powers of the scaled coordinate:
@@ -218,9 +223,11 @@ __device__ __forceinline__ void moment(const double* M, int l, int m, double& re
 
 // Moments of a tile and, from them, the coefficients A, B of Re E_m and Im E_m per (n, m) and
 // quantity that the data kernel multiplies with h_{n,m}: gz; for gz + FTG gz, Uzz, Uxx - Uyy,
-// 2 Uxy, Uxz, Uyz.  Also the tile's own corner weights for the near sum.
+// 2 Uxy, Uxz, Uyz.  Also the tile's own corner weights for the near sum.  grid: x = tiles,
+// y = models.
 template <int MASK>
-__global__ __launch_bounds__(kBlock) void k_tile_moments(TileGrid g, const double* __restrict__ rho,
+__global__ __launch_bounds__(kBlock) void k_tile_moments(TileGrid g, int ntiles,
+                                                         const double* __restrict__ rho, long ld,
                                                          const double* __restrict__ ref,
                                                          HarmonicTable h,
                                                          double* __restrict__ coefs,
@@ -233,6 +240,10 @@ __global__ __launch_bounds__(kBlock) void k_tile_moments(TileGrid g, const doubl
   __shared__ double mu[kMono];
   __shared__ double M[kRows];
   const int t = blockIdx.x;
+  rho += blockIdx.y * ld;
+  ref += blockIdx.y;
+  coefs += (long)blockIdx.y * ntiles * kNM * 2 * NQ;
+  wt += (long)blockIdx.y * ntiles * kTCorners;
   const Tile q = tile_of(g, t);
   axis_moments(g, q, ax);
   for (int e = threadIdx.x; e < kT * kT * kT; e += kBlock) {
@@ -328,7 +339,7 @@ __global__ __launch_bounds__(kBlock) void k_tile_moments(TileGrid g, const doubl
 // 12 (gz: 2) for the sums; bound by the latency of the coefficients' scalar loads (18 KB a tile,
 // more than the scalar cache; 2048 tiles and 4096 sites: gz + FTG 1.9 ms against 0.62 ms of VALU
 // time; gz 0.27 ms, 0.46 ms with one site per lane).  Sums in the corner sums' signs and
-// components: partial[(chunk NC + m) S + s].
+// components: partial[model ld + (chunk NC + m) S + s]; grid: z = models.
 constexpr int kSites = 2;
 // entry of (n, m) in a tile's coefficients
 __host__ __device__ constexpr int entry_nm(int n, int m) {
@@ -400,11 +411,14 @@ template <int MASK>
 __global__ __launch_bounds__(kBlock) void k_tile_far_forward(
     const double* __restrict__ sx, const double* __restrict__ sy, const double* __restrict__ sz,
     int S, const double4* __restrict__ geo, const double* __restrict__ coefs, int ntiles,
-    int per, double* __restrict__ partial) {
+    int per, double* __restrict__ partial, long ld) {
   constexpr int NC = Ncomp<MASK>::value;
   constexpr int NQ = MASK == kMaskScalar ? 1 : 6;
   const int s0 = (blockIdx.x * (kBlock / 64) + (threadIdx.x >> 6)) * 64 * kSites +
                  (int)(threadIdx.x & 63);
+  if (s0 - (int)(threadIdx.x & 63) >= S) return;
+  coefs += (long)blockIdx.z * ntiles * kNM * 2 * NQ;
+  partial += blockIdx.z * ld + (long)blockIdx.y * NC * S;
   double px[kSites], py[kSites], pz[kSites];
   FarSites<NQ> f;
 #pragma unroll
@@ -450,28 +464,29 @@ __global__ __launch_bounds__(kBlock) void k_tile_far_forward(
       out[6] = -f.acc[i][5];
     }
 #pragma unroll
-    for (int m = 0; m < NC; ++m) partial[((long)blockIdx.y * NC + m) * S + s] = out[m];
+    for (int m = 0; m < NC; ++m) partial[(long)m * S + s] = out[m];
   }
 }
 
 // Data, near tiles: a workgroup per site (and split of the tiles); its waves test 64 tiles at a
 // time and share the corners of each near one (tiles dealt to the waves instead left half of
-// them idle: the near ones of a site lie in few runs of 64).  Sums to row `split` of partial.
-template <int MASK>
+// them idle: the near ones of a site lie in few runs of 64).  NB models share the corner terms.
+// Sums to row `split` of partial.
+template <int MASK, int NB>
 __global__ __launch_bounds__(kBlock) void k_tile_near_forward(
     const double* __restrict__ sx, const double* __restrict__ sy, const double* __restrict__ sz,
     int S, TileGrid g, const double4* __restrict__ geo, const double* __restrict__ wt, int ntiles,
-    double* __restrict__ partial) {
+    double* __restrict__ partial, long ld) {
   constexpr int NC = Ncomp<MASK>::value;
   constexpr int W = kBlock / 64;
   __shared__ LogTableShared tab;
-  __shared__ double red[NC][W];
+  __shared__ double red[NB * NC][W];
   const LogTable lg = tab.fill();
   const int s = blockIdx.x, wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
   const double px = sx[s], py = sy[s], pz = sz[s];
-  double acc[NC];
+  double acc[NB * NC];
 #pragma unroll
-  for (int m = 0; m < NC; ++m) acc[m] = 0.0;
+  for (int m = 0; m < NB * NC; ++m) acc[m] = 0.0;
   for (int b = (int)blockIdx.y * 64; b < ntiles; b += (int)gridDim.y * 64) {
     bool near = false;
     if (b + lane < ntiles) near = !offset_of(px, py, pz, geo[b + lane]).far();
@@ -488,30 +503,35 @@ __global__ __launch_bounds__(kBlock) void k_tile_near_forward(
         double v[NC];
         corner_terms_f64<MASK>(px - g.Xc[I], py - g.Yc[J], pz - g.Zc[K], v, lg);
 #pragma unroll
-        for (int m = 0; m < NC; ++m) acc[m] = fma(w[q], v[m], acc[m]);
+        for (int n = 0; n < NB; ++n) {
+          const double wn = w[(long)n * ntiles * kTCorners + q];
+#pragma unroll
+          for (int m = 0; m < NC; ++m) acc[n * NC + m] = fma(wn, v[m], acc[n * NC + m]);
+        }
       }
     }
   }
 #pragma unroll
-  for (int m = 0; m < NC; ++m) {
+  for (int m = 0; m < NB * NC; ++m) {
     double v = acc[m];
 #pragma unroll
     for (int off = 32; off > 0; off >>= 1) v += __shfl_xor(v, off, 64);
     if (lane == 0) red[m][wave] = v;
   }
   __syncthreads();
-  if (threadIdx.x < NC) {
+  if (threadIdx.x < NB * NC) {
     const int m = threadIdx.x;
     double v = 0.0;
     for (int x = 0; x < W; ++x) v += red[m][x];
-    partial[((long)blockIdx.y * NC + m) * S + s] = v;
+    partial[m / NC * ld + ((long)blockIdx.y * NC + m % NC) * S + s] = v;
   }
 }
 
 // Gradient, near tiles: thread = corner of the workgroup's tile; each wave tests 64 sites at a
-// time and sums coef F over the near ones.  H[(split ntiles + t) kTCorners + corner].
+// time and sums coef F over the near ones.  NB residual sets (coef[(set S + s) NC + m]) share the
+// corner terms.  H[((split NB + set) ntiles + t) kTCorners + corner].
 constexpr int kNearThreads = 768;
-template <int MASK>
+template <int MASK, int NB>
 __global__ __launch_bounds__(kNearThreads) void k_tile_near_adjoint(
     const double* __restrict__ sx, const double* __restrict__ sy, const double* __restrict__ sz,
     int S, const double* __restrict__ coef, TileGrid g, const double4* __restrict__ geo,
@@ -526,7 +546,9 @@ __global__ __launch_bounds__(kNearThreads) void k_tile_near_adjoint(
   const double cy = g.Yc[min(tj * kT + q / kTC % kTC, g.ny)];
   const double cz = g.Zc[min(tk * kT + q % kTC, g.nz)];
   const double4 centre = geo[t];
-  double h = 0.0;
+  double h[NB];
+#pragma unroll
+  for (int n = 0; n < NB; ++n) h[n] = 0.0;
   for (int b = (int)blockIdx.y * 64; b < S; b += (int)gridDim.y * 64) {
     bool near = false;
     if (b + lane < S) near = !offset_of(sx[b + lane], sy[b + lane], sz[b + lane], centre).far();
@@ -536,13 +558,18 @@ __global__ __launch_bounds__(kNearThreads) void k_tile_near_adjoint(
       mask &= mask - 1;
       double v[NC];
       corner_terms_f64<MASK>(sx[s] - cx, sy[s] - cy, sz[s] - cz, v, lg);
-      const double* cs = coef + (long)s * NC;
 #pragma unroll
-      for (int m = 0; m < NC; ++m) h = fma(cs[m], v[m], h);
+      for (int n = 0; n < NB; ++n) {
+        const double* cs = coef + ((long)n * S + s) * NC;
+#pragma unroll
+        for (int m = 0; m < NC; ++m) h[n] = fma(cs[m], v[m], h[n]);
+      }
     }
   }
   if ((int)threadIdx.x < kTCorners)
-    H[((long)blockIdx.y * ntiles + t) * kTCorners + threadIdx.x] = h;
+#pragma unroll
+    for (int n = 0; n < NB; ++n)
+      H[(((long)blockIdx.y * NB + n) * ntiles + t) * kTCorners + threadIdx.x] = h[n];
 }
 
 // One h recurrence of order MU (none for MU < 0): value at the current n and at n - 1.
@@ -596,6 +623,26 @@ __device__ __forceinline__ void local_degrees(const double* q0, const double (&t
       local_degrees<MASK, M, L + 1>(q0, tm, zr, u, g0, m2, m1, r0, p1, p2, G, T);
     }
   }
+}
+
+// Sums of n values over the wave's 64 lanes, one or none to a lane: at each step a lane passes
+// half of its values to its partner and adds the partner's to the other half (37 exchanges for
+// the 34 values of order 0; each value by itself takes 204, and the far gradient of 2048 tiles and
+// 256 sites 0.45 ms instead of 0.23).  The same additions as a butterfly of each value.  The lane's sum ends in v[0];
+// returns its index, -1 for none.
+template <int N, int OFF = 32>
+__device__ __forceinline__ int sum_lanes(double* v, int lane) {
+  constexpr int half = (N + 1) / 2;
+  const bool upper = (lane & OFF) != 0;
+#pragma unroll
+  for (int i = 0; i < half; ++i) {
+    const double a = v[i], b = i + half < N ? v[i + half] : 0.0;
+    v[i] = (upper ? b : a) + __shfl_xor(upper ? a : b, OFF, 64);
+  }
+  int at = 0;
+  if constexpr (OFF > 1) at = sum_lanes<half, OFF / 2>(v, lane);
+  if (at >= 0 && upper) at = at + half < N ? at + half : -1;
+  return at;
 }
 
 // Gradient, far tiles, order M: lane = site, the workgroup's four waves stride through the
@@ -680,21 +727,26 @@ __device__ inline void far_adjoint_order(const double* __restrict__ sx,
     }
     local_degrees<MASK, M, M>(q0, tm, zr, u, g0, m2, m1, r0, p1, p2, G, T);
   }
+  constexpr int count = 2 * (kK - M);
+  double v[count];
 #pragma unroll
   for (int l = M; l < kK; ++l)
 #pragma unroll
     for (int c = 0; c < 2; ++c) {
-      double v = odd_factorial(l + 1) * G[l - M][c];
-      if constexpr (MASK != kMaskScalar) v = fma(odd_factorial(l + 2), T[l - M][c], v);
-#pragma unroll
-      for (int off = 32; off > 0; off >>= 1) v += __shfl_xor(v, off, 64);
-      if (lane == 0) red[wave][2 * (l - M) + c] = v;
+      v[2 * (l - M) + c] = odd_factorial(l + 1) * G[l - M][c];
+      if constexpr (MASK != kMaskScalar)
+        v[2 * (l - M) + c] = fma(odd_factorial(l + 2), T[l - M][c], v[2 * (l - M) + c]);
     }
+  if (wave * 64 < S) {
+    const int e = sum_lanes<count>(v, lane);
+    if (e >= 0) red[wave][e] = v[0];
+  }
   __syncthreads();
-  for (int e = threadIdx.x; e < 2 * (kK - M); e += kBlock) {
-    double v = 0.0;
-    for (int w = 0; w < kBlock / 64; ++w) v += red[w][e];
-    lam[2 * lm_index(M + e / 2, M) + e % 2] = v;
+  const int waves = min(kBlock / 64, (S + 63) / 64);  // the ones with sites
+  for (int e = threadIdx.x; e < count; e += kBlock) {
+    double sum = 0.0;
+    for (int w = 0; w < waves; ++w) sum += red[w][e];
+    lam[2 * lm_index(M + e / 2, M) + e % 2] = sum;
   }
 }
 
@@ -711,7 +763,7 @@ __device__ inline void far_adjoint_select(int m, const double* __restrict__ sx,
   }
 }
 
-// grid: x = tiles, y = orders m
+// grid: x = tiles, y = orders m, z = residual sets
 template <int MASK>
 __global__ __launch_bounds__(kBlock) void k_tile_far_adjoint(
     const double* __restrict__ sx, const double* __restrict__ sy, const double* __restrict__ sz,
@@ -719,16 +771,18 @@ __global__ __launch_bounds__(kBlock) void k_tile_far_adjoint(
     double* __restrict__ lam) {
   __shared__ double red[kBlock / 64][2 * kK];
   const int t = tile_of_block(g, blockIdx.x);
-  far_adjoint_select<MASK, 0>((int)blockIdx.y, sx, sy, sz, S, coef, geo[t], red,
-                              lam + (long)t * kRows);
+  far_adjoint_select<MASK, 0>((int)blockIdx.y, sx, sy, sz, S,
+                              coef + (long)blockIdx.z * S * Ncomp<MASK>::value, geo[t], red,
+                              lam + ((long)blockIdx.z * gridDim.x + t) * kRows);
 }
 
 // Local coefficients -> monomials -> the cells' integrals, plus the near corner sums'
-// differences: the tile's cells of the gradient.
+// differences: the tile's cells of the gradient.  grid: x = tiles, y = residual sets.
 __global__ __launch_bounds__(kBlock) void k_tile_gradient(TileGrid g, const double* __restrict__ lam,
                                                           HarmonicTable h,
                                                           const double* __restrict__ H, int splits,
-                                                          int ntiles, double* __restrict__ grad) {
+                                                          int ntiles, double* __restrict__ grad,
+                                                          long ld) {
   __shared__ double ax[3][kT][kK];
   __shared__ double L[kRows];
   __shared__ double mu[kMono];
@@ -736,11 +790,15 @@ __global__ __launch_bounds__(kBlock) void k_tile_gradient(TileGrid g, const doub
   __shared__ double B[kPairs][kT];
   __shared__ double hs[kTCorners];
   const int t = blockIdx.x;
+  lam += (long)blockIdx.y * ntiles * kRows;
+  H += (long)blockIdx.y * ntiles * kTCorners;
+  grad += blockIdx.y * ld;
   const Tile q = tile_of(g, t);
   axis_moments(g, q, ax);
   for (int r = threadIdx.x; r < kRows; r += kBlock) L[r] = lam[(long)t * kRows + r];
   for (int e = threadIdx.x; e < kTCorners; e += kBlock)
-    hs[e] = sum_strided(0.0, H + (long)t * kTCorners + e, splits, (long)ntiles * kTCorners);
+    hs[e] = sum_strided(0.0, H + (long)t * kTCorners + e, splits,
+                        (long)gridDim.y * ntiles * kTCorners);
   __syncthreads();
   for (int e = threadIdx.x; e < kMono; e += kBlock) {
     double s = 0.0;
@@ -895,10 +953,12 @@ HarmonicTable harmonic_table(const jgm_context* ctx) {
           f.cval.as<const double>()};
 }
 
-// Whether the geometry takes the expansions.  They run every model of a batch by itself, the
-// closed form up to eight models per corner evaluation, and a batch's results are the single
-// call's bit for bit, so the choice must not depend on the batch: the expansions are taken
-// where even eight models in turn cost less than eight sharing their corners.
+// Whether the geometry takes the expansions.  A batch's results are the single call's bit for bit,
+// so the choice must not depend on the batch; with more models the closed form gains, whose corner
+// terms all share, where the expansions share only the near ones.  The line is where four models
+// at a time, data and gradient, take the same: on it eight take up to a quarter more than the
+// closed form would and one half as long (gz + FTG, 128 x 128 x 32 cells, 64 stations: 0.40
+// against 0.74 ms for one model, 1.07 and 1.02 for four, 2.0 and 1.7 for eight).
 bool choose(const jgm_context* ctx, bool tensor) {
   const long N = (long)ncells(ctx), S = (long)ctx->S;
   if (N < 100000 || S < 64) return false;
@@ -939,20 +999,36 @@ bool choose(const jgm_context* ctx, bool tensor) {
         }
   }
   near /= samples;
-  // FP64 operations per site, data and gradient averaged: corner terms 250 (gz 170) and 8
-  // models' sums on them; 4650 (1850) per far tile.  The tile kernels take 1.2 to 1.3 times as
-  // long per operation as the corner kernels (128 x 128 x 64 cells, 4096 sites, one model, one
-  // direction: gz + FTG 31 ms closed form, 4.0 ms tiles; gz 16 and 1.7 ms).
-  const double term = tensor ? 250.0 : 170.0, sums = tensor ? 56.0 : 8.0;
-  const double tile = tensor ? 4650.0 : 1850.0;
-  const double closed = (double)ncorners(ctx) * (term + sums);
-  const double split = 1.3 * 8.0 * (near * kTCorners * (term + sums / 8.0) + (tiles - near) * tile);
+  // In the closed form's FP64 operations per site, data and gradient averaged: corner terms 250
+  // (gz 170) and the four models' sums on them; 4650 (1850) per far tile.  The tile kernels take
+  // twice as long per operation, and a tile of a model its moments, the cells' gradients and the
+  // ends of its sums over the sites, as 3 (2) million operations.  Fitted to 18 geometries of
+  // 128 x 128 x 64 to 128 x 128 x 8 cells and 64 to 4096 sites, with which it agrees within 20 %
+  // (four models, gz + FTG, tiles against the closed form: 128 x 128 x 64 cells and 1024 sites 7.1
+  // and 17.4 ms, 256 sites 2.8 and 4.7, 64 sites 2.0 and 1.7; 64 x 64 x 32 cells and 4096 sites
+  // 6.5 and 9.2, 256 sites 0.91 and 0.85).
+  const double term = tensor ? 250.0 + 28.0 : 170.0 + 4.0;
+  const double tile = tensor ? 4650.0 : 1850.0, ends = tensor ? 2.9e6 : 1.9e6;
+  const double closed = (double)ncorners(ctx) * term;
+  const double split = 2.0 * (near * kTCorners * term + 4.0 * (tiles - near) * tile) +
+                       4.0 * tiles * ends / (double)S;
   return split < closed;
 }
 
+// The calls of a launch over nb in {1, 2, 4, 8} models, nb a template argument.
+template <class F>
+void with_models(int nb, F&& f) {
+  switch (nb) {
+    case 8: f(std::integral_constant<int, 8>()); break;
+    case 4: f(std::integral_constant<int, 4>()); break;
+    case 2: f(std::integral_constant<int, 2>()); break;
+    default: f(std::integral_constant<int, 1>()); break;
+  }
+}
+
 template <int MASK>
-hipError_t forward_partials(jgm_context* ctx, const double* model, double** partial,
-                            int* nchunks) {
+hipError_t forward_partials(jgm_context* ctx, int nb, const double* models, size_t model_ld,
+                            double** partial, int* nchunks) {
   constexpr int NC = Ncomp<MASK>::value;
   constexpr int NQ = MASK == kMaskScalar ? 1 : 6;
   TileFar& f = ctx->tile_far;
@@ -960,42 +1036,45 @@ hipError_t forward_partials(jgm_context* ctx, const double* model, double** part
   const TileGrid g = tile_grid(ctx);
   const int ntiles = g.tx * g.ty * g.tz, S = (int)ctx->S;
   // far: chunks of tiles for about 16 waves per SIMD; near: a split per 1024 sites short of
-  // filling the CUs
+  // filling the CUs; neither depends on the number of models, whose sums must not either
   const int site_blocks = (int)blocks_for(S), far_blocks = (int)blocks_for((S + kSites - 1) / kSites);
   const int want = std::max(1, std::min(ntiles, 16 * ctx->cu_count / far_blocks));
   const int per = (ntiles + want - 1) / want, far_chunks = (ntiles + per - 1) / per;
   const int splits = std::max(1, std::min(8, 2048 / S));
   hipError_t e;
-  if ((e = f.coefs.ensure(sizeof(double) * (size_t)ntiles * kNM * 2 * NQ)) != hipSuccess ||
-      (e = f.wt.ensure(sizeof(double) * (size_t)ntiles * kTCorners)) != hipSuccess ||
-      (e = f.ref.ensure(sizeof(double))) != hipSuccess ||
-      (e = ctx->partial.ensure(sizeof(double) * (size_t)(far_chunks + splits + 1) * NC * S)) !=
+  if ((e = f.coefs.ensure(sizeof(double) * (size_t)nb * ntiles * kNM * 2 * NQ)) != hipSuccess ||
+      (e = f.wt.ensure(sizeof(double) * (size_t)nb * ntiles * kTCorners)) != hipSuccess ||
+      (e = f.ref.ensure(sizeof(double) * 8)) != hipSuccess ||
+      (e = ctx->partial.ensure(sizeof(double) * (size_t)(far_chunks + splits + 1) * nb * NC * S)) !=
           hipSuccess)
     return e;
   const double *sx = ctx->d_sx.as<const double>(), *sy = ctx->d_sy.as<const double>(),
                *sz = ctx->d_sz.as<const double>();
+  const long row = (long)NC * S, ld = (far_chunks + splits + 1) * row;  // of a model
   double* part = ctx->partial.as<double>();
   {
     ProfScope ps(ctx, "tile_moments_fp64");
-    hipLaunchKernelGGL(k_reference_density, dim3(1), dim3(1024), 0, st, model,
+    hipLaunchKernelGGL(k_reference_density, dim3(nb), dim3(1024), 0, st, models, (long)model_ld,
                        (long)ncells(ctx), f.ref.as<double>());
     hipLaunchKernelGGL((k_reference_box<MASK>), dim3(site_blocks), dim3(kBlock), 0, st, sx, sy, sz,
-                       S, g, f.ref.as<const double>(),
-                       part + (size_t)(far_chunks + splits) * NC * S);
-    hipLaunchKernelGGL((k_tile_moments<MASK>), dim3(ntiles), dim3(kBlock), 0, st, g, model,
-                       f.ref.as<const double>(), harmonic_table(ctx), f.coefs.as<double>(), f.wt.as<double>());
+                       S, g, f.ref.as<const double>(), nb, part + (far_chunks + splits) * row, ld);
+    hipLaunchKernelGGL((k_tile_moments<MASK>), dim3(ntiles, nb), dim3(kBlock), 0, st, g, ntiles,
+                       models, (long)model_ld, f.ref.as<const double>(), harmonic_table(ctx),
+                       f.coefs.as<double>(), f.wt.as<double>());
   }
   {
     ProfScope ps(ctx, "tile_far_forward_fp64");
-    hipLaunchKernelGGL((k_tile_far_forward<MASK>), dim3(far_blocks, far_chunks), dim3(kBlock), 0,
-                       st, sx, sy, sz, S, f.geo.as<const double4>(), f.coefs.as<const double>(),
-                       ntiles, per, part);
+    hipLaunchKernelGGL((k_tile_far_forward<MASK>), dim3(far_blocks, far_chunks, nb), dim3(kBlock),
+                       0, st, sx, sy, sz, S, f.geo.as<const double4>(),
+                       f.coefs.as<const double>(), ntiles, per, part, ld);
   }
   {
     ProfScope ps(ctx, "tile_near_forward_fp64");
-    hipLaunchKernelGGL((k_tile_near_forward<MASK>), dim3(S, splits), dim3(kBlock), 0, st, sx, sy,
-                       sz, S, g, f.geo.as<const double4>(), f.wt.as<const double>(), ntiles,
-                       part + (size_t)far_chunks * NC * S);
+    with_models(nb, [&](auto n) {
+      hipLaunchKernelGGL((k_tile_near_forward<MASK, decltype(n)::value>), dim3(S, splits),
+                         dim3(kBlock), 0, st, sx, sy, sz, S, g, f.geo.as<const double4>(),
+                         f.wt.as<const double>(), ntiles, part + far_chunks * row, ld);
+    });
   }
   *partial = part;
   *nchunks = far_chunks + splits + 1;
@@ -1003,34 +1082,38 @@ hipError_t forward_partials(jgm_context* ctx, const double* model, double** part
 }
 
 template <int MASK>
-hipError_t adjoint_cells(jgm_context* ctx, const double* coef, double* grad) {
+hipError_t adjoint_cells(jgm_context* ctx, int nb, const double* coef, double* grads,
+                         size_t grad_ld) {
   TileFar& f = ctx->tile_far;
   hipStream_t st = ctx->stream;
   const TileGrid g = tile_grid(ctx);
   const int ntiles = g.tx * g.ty * g.tz, S = (int)ctx->S;
   const int splits = std::max(1, std::min(4, S / 256));
   hipError_t e;
-  if ((e = f.lam.ensure(sizeof(double) * (size_t)ntiles * kRows)) != hipSuccess ||
-      (e = ctx->hpart.ensure(sizeof(double) * (size_t)splits * ntiles * kTCorners)) != hipSuccess)
+  if ((e = f.lam.ensure(sizeof(double) * (size_t)nb * ntiles * kRows)) != hipSuccess ||
+      (e = ctx->hpart.ensure(sizeof(double) * (size_t)splits * nb * ntiles * kTCorners)) !=
+          hipSuccess)
     return e;
   const double *sx = ctx->d_sx.as<const double>(), *sy = ctx->d_sy.as<const double>(),
                *sz = ctx->d_sz.as<const double>();
   {
     ProfScope ps(ctx, "tile_far_adjoint_fp64");
-    hipLaunchKernelGGL((k_tile_far_adjoint<MASK>), dim3(ntiles, kK), dim3(kBlock), 0, st, sx, sy,
-                       sz, S, coef, g, f.geo.as<const double4>(), f.lam.as<double>());
+    hipLaunchKernelGGL((k_tile_far_adjoint<MASK>), dim3(ntiles, kK, nb), dim3(kBlock), 0, st, sx,
+                       sy, sz, S, coef, g, f.geo.as<const double4>(), f.lam.as<double>());
   }
   {
     ProfScope ps(ctx, "tile_near_adjoint_fp64");
-    hipLaunchKernelGGL((k_tile_near_adjoint<MASK>), dim3(ntiles, splits), dim3(kNearThreads), 0,
-                       st, sx, sy, sz, S, coef, g, f.geo.as<const double4>(), ntiles,
-                       ctx->hpart.as<double>());
+    with_models(nb, [&](auto n) {
+      hipLaunchKernelGGL((k_tile_near_adjoint<MASK, decltype(n)::value>), dim3(ntiles, splits),
+                         dim3(kNearThreads), 0, st, sx, sy, sz, S, coef, g,
+                         f.geo.as<const double4>(), ntiles, ctx->hpart.as<double>());
+    });
   }
   {
     ProfScope ps(ctx, "tile_gradient_fp64");
-    hipLaunchKernelGGL(k_tile_gradient, dim3(ntiles), dim3(kBlock), 0, st, g,
+    hipLaunchKernelGGL(k_tile_gradient, dim3(ntiles, nb), dim3(kBlock), 0, st, g,
                        f.lam.as<const double>(), harmonic_table(ctx),
-                       ctx->hpart.as<const double>(), splits, ntiles, grad);
+                       ctx->hpart.as<const double>(), splits, ntiles, grads, (long)grad_ld);
   }
   return hipGetLastError();
 }
@@ -1076,15 +1159,28 @@ hipError_t tile_far_prepare(jgm_context* ctx, int kind, bool* applies) {
   return hipSuccess;
 }
 
-hipError_t tile_far_forward(jgm_context* ctx, int kind, const double* model, double** partial,
-                            int* nchunks) {
-  return kind == JGM_KIND_SCALAR ? forward_partials<kMaskScalar>(ctx, model, partial, nchunks)
-                                 : forward_partials<kMaskAll>(ctx, model, partial, nchunks);
+// Models to a launch of the up to `left` that remain: the moments of one take 15 KB (gz + FTG) a
+// tile, so a mesh of 2^26 cells takes 2 GiB at a time, one of 2^29 cells in turn.
+int tile_far_models(const jgm_context* ctx, int kind, size_t left) {
+  const TileGrid g = tile_grid(ctx);
+  const size_t one = sizeof(double) * kNM * (kind == JGM_KIND_SCALAR ? 2 : 12) * (size_t)g.tx *
+                     g.ty * g.tz;
+  int nb = left >= 8 ? 8 : left >= 4 ? 4 : left >= 2 ? 2 : 1;
+  while (nb > 1 && nb * one > (size_t)2 << 30) nb /= 2;
+  return nb;
 }
 
-hipError_t tile_far_adjoint(jgm_context* ctx, int kind, const double* coef, double* grad) {
-  return kind == JGM_KIND_SCALAR ? adjoint_cells<kMaskScalar>(ctx, coef, grad)
-                                 : adjoint_cells<kMaskAll>(ctx, coef, grad);
+hipError_t tile_far_forward(jgm_context* ctx, int kind, int nb, const double* models,
+                            size_t model_ld, double** partial, int* nchunks) {
+  return kind == JGM_KIND_SCALAR
+             ? forward_partials<kMaskScalar>(ctx, nb, models, model_ld, partial, nchunks)
+             : forward_partials<kMaskAll>(ctx, nb, models, model_ld, partial, nchunks);
+}
+
+hipError_t tile_far_adjoint(jgm_context* ctx, int kind, int nb, const double* coef, double* grads,
+                            size_t grad_ld) {
+  return kind == JGM_KIND_SCALAR ? adjoint_cells<kMaskScalar>(ctx, nb, coef, grads, grad_ld)
+                                 : adjoint_cells<kMaskAll>(ctx, nb, coef, grads, grad_ld);
 }
 
 }  // namespace jgm

@@ -136,15 +136,16 @@ def test_uniform_mesh_is_one_box():
     check_data(ctx, mv, got, closed_form(ctx, KIND["joint"], mv, got.size), "joint")
 
 
+@pytest.mark.parametrize("count", [3, 8, 15])  # launches of 2 + 1, 8 and 8 + 4 + 2 + 1
 @pytest.mark.parametrize("kind", ["gz", "joint"])
-def test_batches_equal_single_calls(kind):
+def test_batches_equal_single_calls(kind, count):
     dims, nsites = ((100, 99, 61), 333) if kind == "gz" else ((125, 119, 61), 260)
     ctx, mv, rng = setup(kind, dims, 1.0, nsites)
     K, k = KIND[kind], 1 if kind == "gz" else 10
-    M = mv[None, :] * (1 + 0.01 * rng.normal(size=(3, 1)))
-    R = rng.normal(size=(3, nsites * k))
+    M = mv[None, :] * (1 + 0.01 * rng.normal(size=(count, 1)))
+    R = rng.normal(size=(count, nsites * k))
     F, G = ctx.forward_batch(K, nat.FP64, M), ctx.adjoint_batch(K, nat.FP64, None, R)
-    for b in range(3):
+    for b in range(count):
         assert np.array_equal(F[b], ctx.forward(K, nat.FP64, M[b]))
         assert np.array_equal(G[b], ctx.adjoint(K, nat.FP64, None, R[b]))
 
