@@ -961,15 +961,18 @@ HarmonicTable harmonic_table(const jgm_context* ctx) {
 // against 0.74 ms for one model, 1.07 and 1.02 for four, 2.0 and 1.7 for eight).
 bool choose(const jgm_context* ctx, bool tensor) {
   const long N = (long)ncells(ctx), S = (long)ctx->S;
-  if (N < 100000 || S < 64) return false;
-  // increasing corner coordinates (the tiles' boxes), and no station with two coordinates on
-  // corner planes: on a mesh line the closed form's guarded logarithms are not the field
+  // not measured below; 48 x 48 x 24 cells, where most tiles are near, lose (600 sites 0.90 ms, tiles
+  // 1.2 ms for four models)
+  if (N < 50000 || S < 64) return false;
+  // increasing corner coordinates (the tiles' boxes), and with the tensor no station with two
+  // coordinates on corner planes: on a mesh line the closed form's guarded logarithms are not the
+  // field.  (In gz a factor of zero stands before them.)
   const std::vector<double>* C[3] = {&ctx->xc, &ctx->yc, &ctx->zc};
   for (const auto* c : C)
     for (size_t i = 1; i < c->size(); ++i)
       if (!((*c)[i] > (*c)[i - 1])) return false;
   const std::vector<double>* P[3] = {&ctx->hsx, &ctx->hsy, &ctx->hsz};
-  for (long s = 0; s < S; ++s) {
+  for (long s = 0; tensor && s < S; ++s) {
     int on = 0;
     for (int a = 0; a < 3; ++a) on += std::binary_search(C[a]->begin(), C[a]->end(), (*P[a])[s]);
     if (on >= 2) return false;

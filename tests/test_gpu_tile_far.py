@@ -16,7 +16,7 @@ from jif3d_amd.model import ThreeDGravityModel, TensorGravityData
 
 pytestmark = pytest.mark.gpu
 KIND = {"gz": nat.KIND_SCALAR, "joint": nat.KIND_SCALAR_TENSOR}
-CASES = [("gz", (100, 99, 61), 1.0, 333), ("gz", (127, 101, 63), 1.03, 700),
+CASES = [("gz", (100, 99, 61), 1.0, 333), ("gz", (64, 61, 31), 1.0, 1000), ("gz", (127, 101, 63), 1.03, 700),
          ("joint", (125, 119, 61), 1.0, 260), ("joint", (128, 128, 64), 1.0, 130)]
 
 
@@ -136,6 +136,22 @@ def test_uniform_mesh_is_one_box():
     check_data(ctx, mv, got, closed_form(ctx, KIND["joint"], mv, got.size), "joint")
 
 
+def test_gz_of_a_station_on_a_mesh_line():
+    """The guarded logarithms of the closed form carry a factor of zero in gz."""
+    ctx, mv, rng = setup("gz", (100, 99, 61), 1.0, 333, on_line=True)
+    assert "tile_far_forward_fp64" in kernels(ctx, lambda: ctx.forward(KIND["gz"], nat.FP64, mv))
+    check_data(ctx, mv, ctx.forward(KIND["gz"], nat.FP64, mv),
+               closed_form(ctx, KIND["gz"], mv, 333), "gz")
+    r = np.zeros(333)
+    r[5] = 1.0
+    g, rows = ctx.adjoint(KIND["gz"], nat.FP64, None, r), ctx.alloc((1, mv.size))
+    ctx.sensitivity_rows(KIND["gz"], 5, 1, rows)
+    ctx.synchronize()
+    ref = 2.0 * rows.to_host()[0]
+    rows.free()
+    assert np.max(np.abs(g - ref)[:-2]) <= 1e-10 * np.max(np.abs(ref[:-2]))
+
+
 @pytest.mark.parametrize("count", [3, 8, 15])  # launches of 2 + 1, 8 and 8 + 4 + 2 + 1
 @pytest.mark.parametrize("kind", ["gz", "joint"])
 def test_batches_equal_single_calls(kind, count):
@@ -151,10 +167,10 @@ def test_batches_equal_single_calls(kind, count):
 
 
 def test_where_the_closed_form_stays():
-    """A station on a mesh line, a small mesh, and the tensor kind keep the closed form."""
-    ctx, mv, _ = setup("gz", (100, 99, 61), 1.0, 333, on_line=True)
-    names = kernels(ctx, lambda: ctx.forward(KIND["gz"], nat.FP64, mv))
-    assert "forward_corners_fp64_gz" in names and "tile_far_forward_fp64" not in names
+    """A tensor station on a mesh line, a small mesh, and the tensor kind keep the closed form."""
+    ctx, mv, _ = setup("joint", (125, 119, 61), 1.0, 260, on_line=True)
+    names = kernels(ctx, lambda: ctx.forward(KIND["joint"], nat.FP64, mv))
+    assert "forward_corners_fp64_gz_ftg" in names and "tile_far_forward_fp64" not in names
     ctx, mv, _ = setup("gz", (30, 30, 20), 1.0, 100)
     assert "forward_corners_fp64_gz" in kernels(ctx, lambda: ctx.forward(KIND["gz"], nat.FP64, mv))
     ctx, mv, _ = setup("gz", (100, 99, 61), 1.0, 333)
