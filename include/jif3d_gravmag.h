@@ -64,7 +64,7 @@ typedef enum jgm_kind {
   JGM_KIND_MAGNETIZATION = 6
 } jgm_kind;
 
-/* JGM_FP64: closed-form box terms in FP64 for every site-cell pair.  From 50000 cells
+/* JGM_FP64: closed-form box terms in FP64 for every site-cell pair.  From 60000 cells
  * (where it is faster for four models at a time; with the tensor, sites off the mesh lines) the
  * scalar and scalar+tensor kinds sum tiles of 8 x 8 x 8 cells farther than 4 of their half-diagonals by
  * FP64 solid-harmonic expansions of degree 16: within 1e-12 of each component's largest value

@@ -334,12 +334,12 @@ __global__ __launch_bounds__(kBlock) void k_tile_moments(TileGrid g, int ntiles,
 }
 
 // Data, far tiles: a lane has kSites sites (64 apart), a workgroup of four waves walks a chunk of
-// tiles, their coefficients wave-uniform (scalar loads).  Orders m outermost, so a lane holds one
-// h recurrence and the 2 NQ sums of the order per site.  3 FP64 operations per (n, m) for h and
-// 12 (gz: 2) for the sums; bound by the latency of the coefficients' scalar loads (18 KB a tile,
-// more than the scalar cache; 2048 tiles and 4096 sites: gz + FTG 1.9 ms against 0.62 ms of VALU
-// time; gz 0.27 ms, 0.46 ms with one site per lane).  Sums in the corner sums' signs and
-// components: partial[model ld + (chunk NC + m) S + s]; grid: z = models.
+// tiles.  The tile's coefficients (18 KB, gz 3 KB) go through LDS, the next tile's on their way in
+// registers: as scalar loads, which the scalar cache does not hold, their latency took twice the
+// rest (2048 tiles and 4096 sites, gz + FTG: 0.83 ms, 1.90 ms with scalar loads; 0.62 ms is
+// the VALU's).  Orders m outermost, so a lane holds one h recurrence and the 2 NQ sums of the order
+// per site: 3 FP64 operations per (n, m) for h and 12 (gz: 2) for the sums.  Sums in the corner
+// sums' signs and components: partial[model ld + (chunk NC + m) S + s]; grid: z = models.
 constexpr int kSites = 2;
 // entry of (n, m) in a tile's coefficients
 __host__ __device__ constexpr int entry_nm(int n, int m) {
@@ -416,9 +416,11 @@ __global__ __launch_bounds__(kBlock) void k_tile_far_forward(
   constexpr int NQ = MASK == kMaskScalar ? 1 : 6;
   const int s0 = (blockIdx.x * (kBlock / 64) + (threadIdx.x >> 6)) * 64 * kSites +
                  (int)(threadIdx.x & 63);
-  if (s0 - (int)(threadIdx.x & 63) >= S) return;
   coefs += (long)blockIdx.z * ntiles * kNM * 2 * NQ;
   partial += blockIdx.z * ld + (long)blockIdx.y * NC * S;
+  constexpr int kPieces = kNM * NQ, kLoads = (kPieces + kBlock - 1) / kBlock;  // of 16 bytes
+  __shared__ double2 tile[2][kPieces];
+  const bool busy = s0 - (int)(threadIdx.x & 63) < S;  // the wave has sites
   double px[kSites], py[kSites], pz[kSites];
   FarSites<NQ> f;
 #pragma unroll
@@ -431,7 +433,24 @@ __global__ __launch_bounds__(kBlock) void k_tile_far_forward(
     for (int v = 0; v < NQ; ++v) f.acc[i][v] = 0.0;
   }
   const int t0 = blockIdx.y * per, t1 = min(t0 + per, ntiles);
+  double2 next[kLoads];
+  auto load = [&](int t) {
+    const double2* from = reinterpret_cast<const double2*>(coefs) + (long)t * kPieces;
+#pragma unroll
+    for (int l = 0; l < kLoads; ++l)
+      next[l] = from[min(l * kBlock + (int)threadIdx.x, kPieces - 1)];
+  };
+  auto store = [&](int buf) {
+#pragma unroll
+    for (int l = 0; l < kLoads; ++l)
+      if (l * kBlock + (int)threadIdx.x < kPieces) tile[buf][l * kBlock + threadIdx.x] = next[l];
+  };
+  load(t0);
+  store(0);
+  __syncthreads();
   for (int t = t0; t < t1; ++t) {
+    const int buf = (t - t0) & 1;
+    if (t + 1 < t1) load(t + 1);
     const double4 centre = geo[t];
     bool any = false;
 #pragma unroll
@@ -446,8 +465,9 @@ __global__ __launch_bounds__(kBlock) void k_tile_far_forward(
       f.er[i] = sqrt(f.u[i]);  // E_0
       f.ei[i] = 0.0;
     }
-    if (!any) continue;
-    far_orders<NQ, 0>(coefs + (long)t * kNM * 2 * NQ, f);
+    if (busy && __any(any)) far_orders<NQ, 0>(reinterpret_cast<const double*>(tile[buf]), f);
+    if (t + 1 < t1) store(buf ^ 1);
+    __syncthreads();
   }
 #pragma unroll
   for (int i = 0; i < kSites; ++i) {
@@ -957,13 +977,13 @@ HarmonicTable harmonic_table(const jgm_context* ctx) {
 // so the choice must not depend on the batch; with more models the closed form gains, whose corner
 // terms all share, where the expansions share only the near ones.  The line is where four models
 // at a time, data and gradient, take the same: on it eight take up to a quarter more than the
-// closed form would and one half as long (gz + FTG, 128 x 128 x 32 cells, 64 stations: 0.40
-// against 0.74 ms for one model, 1.07 and 1.02 for four, 2.0 and 1.7 for eight).
+// closed form would and one half as long (gz + FTG, 128 x 128 x 32 cells, 64 stations: 0.36
+// against 0.73 ms for one model, 1.00 and 1.04 for four, 1.8 and 1.7 for eight).
 bool choose(const jgm_context* ctx, bool tensor) {
   const long N = (long)ncells(ctx), S = (long)ctx->S;
-  // not measured below; 48 x 48 x 24 cells, where most tiles are near, lose (600 sites 0.90 ms, tiles
-  // 1.2 ms for four models)
-  if (N < 50000 || S < 64) return false;
+  // 48 x 48 x 24 cells, where most tiles are near, lose (gz of 625 sites, four models 0.60 ms,
+  // closed form 0.53), 128 x 64 x 8 win (4096 sites 1.2 and 2.5 ms)
+  if (N < 60000 || S < 64) return false;
   // increasing corner coordinates (the tiles' boxes), and with the tensor no station with two
   // coordinates on corner planes: on a mesh line the closed form's guarded logarithms are not the
   // field.  (In gz a factor of zero stands before them.)
@@ -1003,18 +1023,18 @@ bool choose(const jgm_context* ctx, bool tensor) {
   }
   near /= samples;
   // In the closed form's FP64 operations per site, data and gradient averaged: corner terms 250
-  // (gz 170) and the four models' sums on them; 4650 (1850) per far tile.  The tile kernels take
-  // twice as long per operation, and a tile of a model its moments, the cells' gradients and the
-  // ends of its sums over the sites, as 3 (2) million operations.  Fitted to 18 geometries of
-  // 128 x 128 x 64 to 128 x 128 x 8 cells and 64 to 4096 sites, with which it agrees within 20 %
-  // (four models, gz + FTG, tiles against the closed form: 128 x 128 x 64 cells and 1024 sites 7.1
-  // and 17.4 ms, 256 sites 2.8 and 4.7, 64 sites 2.0 and 1.7; 64 x 64 x 32 cells and 4096 sites
-  // 6.5 and 9.2, 256 sites 0.91 and 0.85).
+  // (gz 170) and the four models' sums on them, 4650 (1850) per far tile.  The near kernels take
+  // twice as long per operation, the far ones 1.3 (2) times; a tile of a model its moments, the
+  // cells' gradients and the ends of its sums over the sites, as 2.3 (1.75) million operations; the
+  // launches of either form 5 to 9 thousand million.  Fitted to 26 geometries of 128 x 128 x 64 to
+  // 48 x 48 x 24 cells and 36 to 4096 sites (four models, gz + FTG, tiles against the closed form:
+  // 128 x 128 x 64 cells and 1024 sites 5.3 and 17.3 ms, 256 sites 2.3 and 4.6, 64 sites 1.8 and
+  // 1.7; 64 x 64 x 32 cells and 4096 sites 5.9 and 9.1, 256 sites 0.88 and 0.85).
   const double term = tensor ? 250.0 + 28.0 : 170.0 + 4.0;
-  const double tile = tensor ? 4650.0 : 1850.0, ends = tensor ? 2.9e6 : 1.9e6;
-  const double closed = (double)ncorners(ctx) * term;
-  const double split = 2.0 * (near * kTCorners * term + 4.0 * (tiles - near) * tile) +
-                       4.0 * tiles * ends / (double)S;
+  const double far_tile = tensor ? 1.3 * 4650.0 : 2.0 * 1850.0, ends = tensor ? 2.3e6 : 1.75e6;
+  const double closed = (double)ncorners(ctx) * term + (tensor ? 6.0e9 : 9.4e9) / (double)S;
+  const double split = 2.2 * near * kTCorners * term + 4.0 * (tiles - near) * far_tile +
+                       (4.0 * tiles * ends + 4.8e9) / (double)S;
   return split < closed;
 }
 
