@@ -1415,7 +1415,9 @@ hipError_t forward_mixed_impl(jgm_context* ctx, int kind, int nbm, const double*
   if ((e = ctx->nearpart.ensure(sizeof(double) * (size_t)nbm * S * NC)) != hipSuccess) return e;
   if (N > 0) {
     const int site_blocks = (S + kBlock - 1) / kBlock;
-    const long waves_per_chunk = (S + 63) / 64;
+    // counted with the waves that have no site and end at once: a finer cut of 2401 sites' tiles
+    // (5 instead of 6 a chunk, magnetization, 75 x 106 x 61 cells) took 8.77 instead of 8.69 ms
+    const long waves_per_chunk = (long)site_blocks * (kBlock / 64);
     long want = (ctx->far_fwd_waves + waves_per_chunk - 1) / waves_per_chunk;
     want = std::max<long>(1, std::min<long>(want, ntiles));
     const long per = (ntiles + want - 1) / want;
