@@ -113,7 +113,7 @@ struct SlabMesh {
 struct TileFar {
   unsigned long gen[2] = {0, 0}, geo_gen = 0;
   bool chosen[2] = {false, false}, tables = false;
-  DeviceBuffer ptr, idx, cptr, cidx, mono, val, cval, geo, coefs, wt, ref, lam;
+  DeviceBuffer table, geo, coefs, wt, ref, lam;
 };
 
 // Optional per-kernel timing: HIP events recorded on the context's stream around
