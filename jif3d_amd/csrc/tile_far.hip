@@ -14,13 +14,19 @@
 // The gradient is the transpose: local coefficients Lambda_l^m per tile, summed over the far
 // sites, then integrated over each cell as a polynomial.
 //
-// Truncation: the terms left out are below (1/4)^17 of a tile's field where it is nearest and
-// fall with the 17th power of its distance; tiles of log-normal, noisy or uniform densities
-// leave 5e-14 of the nearest tile's gz and 6e-13 of its Uzz.  The closed form that it replaces
-// rounds each far term to about 1e-16 (d/a)^3 of itself, so the sums are no less accurate.
+// Truncation: it is largest for a body of one cell in a corner of its tile, seen in that corner's
+// direction from kRatio half-diagonals.  Of the body's largest value at that distance it is at most
+// 9e-13 there, in every tensor component and in gz, for tiles of any shape (1 to 8 cells a side,
+// cells of 1 : 4 to 4 : 1); 2 x 2 x 2 cells of a whole tile leave 2e-13, 4 x 4 x 4 2e-14, the tile
+// itself 2e-15.  The closed form's own rounding is no smaller: 8e-13 to 2e-12 (median over
+// directions) of one cell's diagonal components there, 5e-12 of the others, 1e-11 of gz, and less
+// as the body grows.  So no density loses accuracy to the expansions.  (Degree 16 from 4
+// half-diagonals on takes 6.8 instead of 9.4 ms for data and gradient of 2048 tiles and 4096 sites,
+// but leaves 6e-10 of one cell and 1e-11 of 4 x 4 x 4; degree 22 from 4 on takes 9.3 ms, but 16.4
+// instead of 14.2 for eight models and 1024 sites.)
 //
-// A site-tile pair takes about 3200 FP64 operations (gz + FTG; 1100 for gz) in the data and 6100
-// (2600) in the gradient, against 512 cells at 250 (170) and as many corners.
+// A site-tile pair takes about 4700 FP64 operations (gz + FTG; 1600 for gz) in the data and 9200
+// (3900) in the gradient, against 512 cells at 250 (170) and as many corners.
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
@@ -41,11 +47,13 @@ constexpr int kBlock = 256;
 constexpr int kT = 8;                       // cells per tile and axis
 constexpr int kTC = kT + 1;                 // corners per tile and axis
 constexpr int kTCorners = kTC * kTC * kTC;  // 729
-constexpr int kDeg = 16;                    // largest degree of the moments
+constexpr int kDeg = 20;                    // largest degree of the moments
 constexpr int kK = kDeg + 1;
-constexpr double kRatio = 4.0;              // nearest far site, in tile half-diagonals
-constexpr int kMono = kK * (kK + 1) * (kK + 2) / 6;  // monomials of degree <= kDeg: 969
-constexpr int kPairs = kK * (kK + 1) / 2;            // (l, m), 0 <= m <= l: 153
+// nearest far site, in tile half-diagonals
+template <int MASK>
+constexpr double kRatio = MASK == kMaskScalar ? 3.95 : 4.4;
+constexpr int kMono = kK * (kK + 1) * (kK + 2) / 6;  // monomials of degree <= kDeg: 1771
+constexpr int kPairs = kK * (kK + 1) / 2;            // (l, m), 0 <= m <= l: 231
 constexpr int kRows = 2 * kPairs;
 // (n, m) of the irregular harmonics: n = 1 .. kDeg + 2, m = 0 .. n, m-major
 constexpr int kOrders = kDeg + 3;
@@ -117,7 +125,10 @@ __global__ __launch_bounds__(kBlock) void k_tile_centres(TileGrid g, int ntiles,
 // kernel decides with these operations, so a pair is near in one pass and far in the other.
 struct Offset {
   double x, y, z, r2;
-  __device__ __forceinline__ bool far() const { return r2 >= kRatio * kRatio; }
+  template <int MASK>
+  __device__ __forceinline__ bool far() const {
+    return r2 >= kRatio<MASK> * kRatio<MASK>;
+  }
 };
 __device__ __forceinline__ Offset offset_of(double px, double py, double pz, double4 c) {
   Offset o;
@@ -334,12 +345,14 @@ __global__ __launch_bounds__(kBlock) void k_tile_moments(TileGrid g, int ntiles,
 }
 
 // Data, far tiles: a lane has kSites sites (64 apart), a workgroup of four waves walks a chunk of
-// tiles.  The tile's coefficients (18 KB, gz 3 KB) go through LDS, the next tile's on their way in
-// registers: as scalar loads, which the scalar cache does not hold, their latency took twice the
-// rest (2048 tiles and 4096 sites, gz + FTG: 0.83 ms, 1.90 ms with scalar loads; 0.62 ms is
-// the VALU's).  Orders m outermost, so a lane holds one h recurrence and the 2 NQ sums of the order
-// per site: 3 FP64 operations per (n, m) for h and 12 (gz: 2) for the sums.  Sums in the corner
-// sums' signs and components: partial[model ld + (chunk NC + m) S + s]; grid: z = models.
+// tiles.  The tile's coefficients (26 KB, gz 4 KB) go through LDS, the next tile's on their way
+// behind the sums (through 100 bytes of scratch a lane for gz + FTG, whose sums leave no
+// registers): as scalar loads, which the scalar cache does not hold, their latency took twice the
+// rest (2048 tiles and 4096 sites, gz + FTG, degree 16: 0.83 ms, 1.90 ms with scalar loads, 0.62 ms
+// is the VALU's; degree 20: 1.25 ms).  Orders m outermost, so a lane holds one h recurrence and the
+// 2 NQ sums of the order per site: 3 FP64 operations per (n, m) for h and 12 (gz: 2) for the sums.
+// Sums in the corner sums' signs and components: partial[model ld + (chunk NC + m) S + s]; grid:
+// z = models.
 constexpr int kSites = 2;
 // entry of (n, m) in a tile's coefficients
 __host__ __device__ constexpr int entry_nm(int n, int m) {
@@ -456,7 +469,7 @@ __global__ __launch_bounds__(kBlock) void k_tile_far_forward(
 #pragma unroll
     for (int i = 0; i < kSites; ++i) {
       const Offset o = offset_of(px[i], py[i], pz[i], centre);
-      const bool far = o.far();
+      const bool far = o.far<MASK>();
       any = any || far;
       f.u[i] = far ? 1.0 / o.r2 : 0.0;  // near: every E is zero
       f.zr[i] = far ? o.z * f.u[i] : 0.0;
@@ -509,7 +522,7 @@ __global__ __launch_bounds__(kBlock) void k_tile_near_forward(
   for (int m = 0; m < NB * NC; ++m) acc[m] = 0.0;
   for (int b = (int)blockIdx.y * 64; b < ntiles; b += (int)gridDim.y * 64) {
     bool near = false;
-    if (b + lane < ntiles) near = !offset_of(px, py, pz, geo[b + lane]).far();
+    if (b + lane < ntiles) near = !offset_of(px, py, pz, geo[b + lane]).far<MASK>();
     unsigned long long mask = __ballot(near);
     while (mask) {
       const int t = b + __builtin_ctzll(mask);
@@ -571,7 +584,7 @@ __global__ __launch_bounds__(kNearThreads) void k_tile_near_adjoint(
   for (int n = 0; n < NB; ++n) h[n] = 0.0;
   for (int b = (int)blockIdx.y * 64; b < S; b += (int)gridDim.y * 64) {
     bool near = false;
-    if (b + lane < S) near = !offset_of(sx[b + lane], sy[b + lane], sz[b + lane], centre).far();
+    if (b + lane < S) near = !offset_of(sx[b + lane], sy[b + lane], sz[b + lane], centre).far<MASK>();
     unsigned long long mask = __ballot(near);
     while (mask) {
       const int s = __builtin_amdgcn_readfirstlane(b + __builtin_ctzll(mask));
@@ -646,10 +659,10 @@ __device__ __forceinline__ void local_degrees(const double* q0, const double (&t
 }
 
 // Sums of n values over the wave's 64 lanes, one or none to a lane: at each step a lane passes
-// half of its values to its partner and adds the partner's to the other half (37 exchanges for
-// the 34 values of order 0; each value by itself takes 204, and the far gradient of 2048 tiles and
-// 256 sites 0.45 ms instead of 0.23).  The same additions as a butterfly of each value.  The lane's sum ends in v[0];
-// returns its index, -1 for none.
+// half of its values to its partner and adds the partner's to the other half (44 exchanges for
+// the 42 values of order 0; each value by itself takes 252, and the far gradient of 2048 tiles and
+// 256 sites, degree 16, 0.45 ms instead of 0.23).  The same additions as a butterfly of each value.
+// The lane's sum ends in v[0]; returns its index, -1 for none.
 template <int N, int OFF = 32>
 __device__ __forceinline__ int sum_lanes(double* v, int lane) {
   constexpr int half = (N + 1) / 2;
@@ -685,7 +698,7 @@ __device__ inline void far_adjoint_order(const double* __restrict__ sx,
   for (int b = wave * 64; b < S; b += kBlock) {
     const int s = min(b + lane, S - 1);
     Offset o = offset_of(sx[s], sy[s], sz[s], centre);
-    const bool far = b + lane < S && o.far();
+    const bool far = b + lane < S && o.far<MASK>();
     if (__ballot(far) == 0) continue;
     double c7[7];
 #pragma unroll
@@ -693,8 +706,8 @@ __device__ inline void far_adjoint_order(const double* __restrict__ sx,
     if (!far) {  // any far offset: the coefficients are zero
       o.x = 0.0;
       o.y = 0.0;
-      o.z = kRatio;
-      o.r2 = kRatio * kRatio;
+      o.z = kRatio<MASK>;
+      o.r2 = kRatio<MASK> * kRatio<MASK>;
     }
     const double u = 1.0 / o.r2, zr = o.z * u, xu = o.x * u, yu = o.y * u;
     double E[M + 3][2];  // E_0 .. E_{M+2}
@@ -997,14 +1010,14 @@ HarmonicTable harmonic_table(const jgm_context* ctx) {
 
 // Whether the geometry takes the expansions.  A batch's results are the single call's bit for bit,
 // so the choice must not depend on the batch; with more models the closed form gains, whose corner
-// terms all share, where the expansions share only the near ones.  The line is where four models
-// at a time, data and gradient, take the same: on it eight take up to a quarter more than the
-// closed form would and one half as long (gz + FTG, 128 x 128 x 32 cells, 64 stations: 0.36
-// against 0.73 ms for one model, 1.00 and 1.04 for four, 1.8 and 1.7 for eight).
+// terms all share, where the expansions share only the near ones.  The line is where three models
+// at a time, data and gradient, take the same: on it one takes 0.4 to 0.7 of the closed form's time
+// and eight up to a third more (gz + FTG, 128 x 128 x 64 cells, 100 stations: 0.93 against 2.19 ms
+// for one model, 1.63 and 2.28 for two, 2.94 and 2.68 for four, 5.43 and 4.18 for eight).
 bool choose(const jgm_context* ctx, bool tensor) {
   const long N = (long)ncells(ctx), S = (long)ctx->S;
-  // 48 x 48 x 24 cells, where most tiles are near, lose (gz of 625 sites, four models 0.60 ms,
-  // closed form 0.53), 128 x 64 x 8 win (4096 sites 1.2 and 2.5 ms)
+  // 48 x 48 x 24 cells, where most tiles are near, lose (gz of 625 sites, four models 0.68 ms,
+  // closed form 0.55), 128 x 64 x 8 win (4096 sites 1.4 and 2.6 ms)
   if (N < 60000 || S < 64) return false;
   // increasing corner coordinates (the tiles' boxes), and with the tensor no station with two
   // coordinates on corner planes: on a mesh line the closed form's guarded logarithms are not the
@@ -1029,6 +1042,7 @@ bool choose(const jgm_context* ctx, bool tensor) {
       half2[a].push_back(0.25 * (hi - lo) * (hi - lo));
     }
   }
+  const double ratio = tensor ? kRatio<kMaskAll> : kRatio<kMaskScalar>;
   const double tiles = (double)centre[0].size() * centre[1].size() * centre[2].size();
   const long samples = std::min<long>(S, 16);
   double near = 0.0;
@@ -1040,23 +1054,24 @@ bool choose(const jgm_context* ctx, bool tensor) {
           const double dx = ctx->hsx[s] - centre[0][i], dy = ctx->hsy[s] - centre[1][j],
                        dz = ctx->hsz[s] - centre[2][k];
           near += dx * dx + dy * dy + dz * dz <
-                  kRatio * kRatio * (half2[0][i] + half2[1][j] + half2[2][k]);
+                  ratio * ratio * (half2[0][i] + half2[1][j] + half2[2][k]);
         }
   }
   near /= samples;
   // In the closed form's FP64 operations per site, data and gradient averaged: corner terms 250
-  // (gz 170) and the four models' sums on them, 4650 (1850) per far tile.  The near kernels take
-  // twice as long per operation, the far ones 1.3 (2) times; a tile of a model its moments, the
-  // cells' gradients and the ends of its sums over the sites, as 2.3 (1.75) million operations; the
-  // launches of either form 5 to 9 thousand million.  Fitted to 26 geometries of 128 x 128 x 64 to
-  // 48 x 48 x 24 cells and 36 to 4096 sites (four models, gz + FTG, tiles against the closed form:
-  // 128 x 128 x 64 cells and 1024 sites 5.3 and 17.3 ms, 256 sites 2.3 and 4.6, 64 sites 1.8 and
-  // 1.7; 64 x 64 x 32 cells and 4096 sites 5.9 and 9.1, 256 sites 0.88 and 0.85).
-  const double term = tensor ? 250.0 + 28.0 : 170.0 + 4.0;
-  const double far_tile = tensor ? 1.3 * 4650.0 : 2.0 * 1850.0, ends = tensor ? 2.3e6 : 1.75e6;
-  const double closed = (double)ncorners(ctx) * term + (tensor ? 6.0e9 : 9.4e9) / (double)S;
-  const double split = 2.2 * near * kTCorners * term + 4.0 * (tiles - near) * far_tile +
-                       (4.0 * tiles * ends + 4.8e9) / (double)S;
+  // (gz 170) and three models' sums on them, 6950 (2750) per far tile and model.  The near kernels
+  // take 1.9 times as long per operation, the far ones 1.8 (2.9) times; a tile of a model its
+  // moments, the cells' gradients and the ends of its sums over the sites, as 2.45 (1.45) million
+  // operations; the launches and the waves they leave idle 7 to 11 thousand million.  Fitted to
+  // 26 geometries of 128 x 128 x 64 to 48 x 48 x 24 cells and 36 to 4096 sites (four models, gz +
+  // FTG, tiles against the closed form: 128 x 128 x 64 cells and 1024 sites 7.9 and 17.3 ms, 256
+  // sites 3.3 and 4.7, 64 sites 2.8 and 1.8; 64 x 64 x 32 cells and 4096 sites 7.7 and 9.1, 1024
+  // sites 2.5 and 2.5, 256 sites 1.2 and 0.9).
+  const double term = tensor ? 250.0 + 21.0 : 170.0 + 3.0;
+  const double far_tile = tensor ? 1.8 * 6950.0 : 2.9 * 2750.0, ends = tensor ? 2.45e6 : 1.45e6;
+  const double closed = (double)ncorners(ctx) * term + (tensor ? 6.6e9 : 11.5e9) / (double)S;
+  const double split = 1.9 * near * kTCorners * term + 3.0 * (tiles - near) * far_tile +
+                       (3.0 * tiles * ends + (tensor ? 8.2e9 : 11.0e9)) / (double)S;
   return split < closed;
 }
 

@@ -1,0 +1,109 @@
+"""The stated accuracy of the FP64 tile expansions (gz, gz + FTG) where they are least accurate:
+a body of one to eight cells in a corner of its tile, every station just beyond the distance from
+which the tile is expanded (an airborne survey), so that nothing nearer hides the truncation.  Data
+and gradient entries against Gauss-Legendre quadrature of the point source's field over the cells,
+within 1e-12 of each component's largest value over the survey."""
+import numpy as np
+import pytest
+
+from jif3d_amd import _native as nat
+from jif3d_amd.model import ThreeDGravityModel, TensorGravityData
+
+pytestmark = pytest.mark.gpu
+KIND = {"gz": nat.KIND_SCALAR, "joint": nat.KIND_SCALAR_TENSOR}
+NEAREST = {"gz": 3.96, "joint": 4.41}  # half-diagonals; the expansions begin at 3.95 and 4.4
+
+
+def airborne(kind, dims, cell, nsites=500):
+    """Stations in every upward direction from the middle tile of the top layer, 1 to 1.15 times
+    the nearest distance away; a tenth of them near the direction of the tile's first corner."""
+    rng = np.random.default_rng(dims[2])
+    m = ThreeDGravityModel()
+    m.SetMeshSize(*dims)
+    m.SetXCellSizes(np.full(dims[0], cell[0]))
+    m.SetYCellSizes(np.full(dims[1], cell[1]))
+    m.SetZCellSizes(np.full(dims[2], cell[2]))
+    m.shape, m.cell = dims, np.array(cell)
+    m.first = np.array([dims[0] // 16 * 8, dims[1] // 16 * 8, 0])  # the tile's first cell
+    half = 4.0 * m.cell
+    v = rng.normal(size=(3, nsites))
+    v[:, ::10] = -half[:, None] / np.linalg.norm(half) + 0.05 * v[:, ::10]
+    v /= np.linalg.norm(v, axis=0)
+    v[2] = -np.abs(v[2])
+    p = (m.first * m.cell + half)[:, None]
+    p = p + v * np.linalg.norm(half) * NEAREST[kind] * rng.uniform(1.0, 1.15, nsites)
+    p[2] = np.minimum(p[2], -1.0)
+    d = TensorGravityData()
+    d.SetMeasurementPoints(*p)
+    ctx = nat.Context()
+    ctx.configure(m, d)
+    return ctx, m, p, rng
+
+
+G = 6.67428e-11
+NODE, WEIGHT = np.polynomial.legendre.leggauss(8)
+
+
+def box(kind, p, lo, size):
+    """Data of unit density in a box, one row per station, as the kind lays them out.  Eight nodes
+    a side, the box's half-diagonal at most a tenth of the distance: (1/10)^16 is left out.  (The
+    closed form of a far box cancels: in 80-bit arithmetic 1e-12 of Uxz where a station looks along
+    an edge.)"""
+    assert np.min(np.linalg.norm(p - (lo + size / 2)[:, None], axis=0)) > 5 * np.linalg.norm(size)
+    x, y, z = (lo[a] + size[a] * (0.5 + 0.5 * NODE) for a in range(3))
+    w = np.einsum("i,j,k->ijk", WEIGHT, WEIGHT, WEIGHT).ravel() * np.prod(size) / 8
+    d = [q.ravel()[None, :] - s[:, None] for q, s in zip(np.meshgrid(x, y, z, indexing="ij"), p)]
+    r2 = sum(v * v for v in d)
+    r3 = r2 * np.sqrt(r2)
+    out = [d[2] / r3]
+    if kind == "joint":
+        out += [3.0 * d[a] * d[b] / (r2 * r3) - (a == b) / r3 for a in range(3) for b in range(3)]
+    return G * np.stack([v @ w for v in out], axis=1)
+
+
+def takes_tiles(ctx, K, mv):
+    ctx.profile_enable(True)
+    ctx.profile_reset()
+    out = ctx.forward(K, nat.FP64, mv)
+    names = set(ctx.profile())
+    ctx.profile_enable(False)
+    return "tile_far_forward_fp64" in names, out
+
+
+CELLS = [(20.0, 20.0, 20.0), (25.0, 25.0, 10.0)]
+
+
+@pytest.mark.parametrize("cells", [1, 2])
+@pytest.mark.parametrize("cell", CELLS)
+@pytest.mark.parametrize("kind", ["gz", "joint"])
+def test_small_body_in_a_tile_corner(kind, cell, cells):
+    ctx, m, p, _ = airborne(kind, (64, 64, 24), cell)
+    rho = np.zeros(m.shape)
+    i, j, k = m.first
+    rho[i:i + cells, j:j + cells, k:k + cells] = 1000.0
+    tiles, out = takes_tiles(ctx, KIND[kind], rho.ravel())
+    assert tiles
+    exact = 1000.0 * box(kind, p, m.first * m.cell, cells * m.cell)
+    error = np.max(np.abs(out.reshape(exact.shape) - exact), axis=0) / np.max(np.abs(exact), axis=0)
+    assert np.all(error <= 1e-12), error
+
+
+@pytest.mark.parametrize("cell", CELLS)
+@pytest.mark.parametrize("kind", ["gz", "joint"])
+def test_gradient_of_a_tile_corner(kind, cell):
+    ctx, m, p, rng = airborne(kind, (64, 64, 24), cell)
+    K = KIND[kind]
+    assert takes_tiles(ctx, K, np.zeros(np.prod(m.shape)))[0]
+    i, j, k = m.first
+    inside = [(0, 0, 0), (1, 0, 0), (1, 1, 1), (3, 4, 2)]
+    J = np.array([box(kind, p, (m.first + c) * m.cell, m.cell) for c in inside])
+    stations = [0, 10, 20, 3, 7]
+    for c in range(J.shape[2]):
+        largest = np.max(np.abs(J[:, :, c]), axis=1)
+        for s in stations:
+            r = np.zeros((p.shape[1], J.shape[2]))
+            r[s, c] = 1.0
+            g = ctx.adjoint(K, nat.FP64, None, r.ravel()).reshape(m.shape)
+            got = np.array([g[i + a, j + b, k + q] for a, b, q in inside])
+            error = np.abs(got - 2.0 * J[:, s, c]) / (2.0 * largest)
+            assert np.all(error <= 1e-12), (c, s, error)
