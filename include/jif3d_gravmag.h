@@ -65,7 +65,8 @@ typedef enum jgm_kind {
 } jgm_kind;
 
 /* JGM_FP64: closed-form box terms in FP64 for every site-cell pair.  From 60000 cells and 64
- * sites (where it is faster for three models at a time; with the tensor, sites off the mesh lines)
+ * sites (where it is faster for three models at a time; with the tensor, no site nearer a mesh line than
+ * 2^-18 of the line's length ahead of it, where the closed form's logarithms are guarded or lost)
  * jgm_forward and jgm_adjoint of the scalar and scalar+tensor kinds sum tiles of 8 x 8 x 8 cells
  * farther than 3.95 (scalar) or 4.4 of their half-diagonals by FP64 solid-harmonic expansions of
  * degree 20.  What these leave out is within 1e-12 of each component's largest value over the

@@ -1019,18 +1019,31 @@ bool choose(const jgm_context* ctx, bool tensor) {
   // 48 x 48 x 24 cells, where most tiles are near, lose (gz of 625 sites, four models 0.68 ms,
   // closed form 0.55), 128 x 64 x 8 win (4096 sites 1.4 and 2.6 ms)
   if (N < 60000 || S < 64) return false;
-  // increasing corner coordinates (the tiles' boxes), and with the tensor no station with two
-  // coordinates on corner planes: on a mesh line the closed form's guarded logarithms are not the
-  // field.  (In gz a factor of zero stands before them.)
+  // increasing corner coordinates (the tiles' boxes)
   const std::vector<double>* C[3] = {&ctx->xc, &ctx->yc, &ctx->zc};
   for (const auto* c : C)
     for (size_t i = 1; i < c->size(); ++i)
       if (!((*c)[i] > (*c)[i - 1])) return false;
+  // With the tensor, no station on or next to a mesh line.  Of the corners down a line at distance
+  // rho, those at u < 0 along it have log(u + r), u + r = rho^2 / 2|u|, formed with an ulp of |u|:
+  // guarded or a few ulps where rho is small, not the field but what the reference computes, and
+  // tiles that are expanded would give the field instead.  At rho = 2^-18 of the farthest |u| (5 mm
+  // for 1.3 km) the argument keeps 15 bits and the closed form is the field with some noise.  (In
+  // gz a factor of rho stands before these logarithms.)
   const std::vector<double>* P[3] = {&ctx->hsx, &ctx->hsy, &ctx->hsz};
   for (long s = 0; tensor && s < S; ++s) {
-    int on = 0;
-    for (int a = 0; a < 3; ++a) on += std::binary_search(C[a]->begin(), C[a]->end(), (*P[a])[s]);
-    if (on >= 2) return false;
+    double plane2[3];  // squared distances to the nearest corner planes
+    for (int a = 0; a < 3; ++a) {
+      const double v = (*P[a])[s];
+      const auto up = std::lower_bound(C[a]->begin(), C[a]->end(), v);
+      double d = up != C[a]->end() ? *up - v : HUGE_VAL;
+      if (up != C[a]->begin()) d = std::min(d, v - up[-1]);
+      plane2[a] = d * d;
+    }
+    for (int a = 0; a < 3; ++a) {
+      const double u = std::max(0.0, C[a]->back() - (*P[a])[s]);
+      if (plane2[(a + 1) % 3] + plane2[(a + 2) % 3] <= 0x1p-36 * u * u) return false;
+    }
   }
   // near tiles of a sample of stations
   std::vector<double> centre[3], half2[3];

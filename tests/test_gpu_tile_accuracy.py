@@ -3,6 +3,8 @@ a body of one to eight cells in a corner of its tile, every station just beyond 
 which the tile is expanded (an airborne survey), so that nothing nearer hides the truncation.  Data
 and gradient entries against Gauss-Legendre quadrature of the point source's field over the cells,
 within 1e-12 of each component's largest value over the survey."""
+import ctypes
+
 import numpy as np
 import pytest
 
@@ -107,3 +109,55 @@ def test_gradient_of_a_tile_corner(kind, cell):
             got = np.array([g[i + a, j + b, k + q] for a, b, q in inside])
             error = np.abs(got - 2.0 * J[:, s, c]) / (2.0 * largest)
             assert np.all(error <= 1e-12), (c, s, error)
+
+
+# Stations on or next to a mesh line.  The tensor's logarithms are guarded or lose their argument
+# there (not the field, but what the reference computes), down the whole line; a sum that takes
+# the near corners so and the far ones from expansions is neither.
+OFFSETS = [0.0, 2.0 ** -47, 1e-12, 1e-9, 1e-7, 1e-6, 1e-5, 1e-4, 1e-3]
+LINES = {"below": lambda m, o: (m.coords[0][2] + o, m.coords[1][3] - o, -30.0),
+         "ahead": lambda m, o: (-50.0, m.coords[1][3] + o, m.coords[2][2] + o / 2)}
+
+
+def near_line(at):
+    rng = np.random.default_rng(3)
+    m = ThreeDGravityModel()
+    m.SetMeshSize(125, 119, 61)
+    m.SetXCellSizes(np.full(125, 20.0))
+    m.SetYCellSizes(np.full(119, 20.0))
+    m.SetZCellSizes(np.full(61, 15.0))
+    n = 260
+    x, y, z = rng.uniform(3, 2500, n), rng.uniform(3, 2380, n), -rng.uniform(3, 60, n)
+    if at:
+        x[5], y[5], z[5] = at(m)
+    d = TensorGravityData()
+    d.SetMeasurementPoints(x, y, z)
+    ctx = nat.Context()
+    ctx.configure(m, d)
+    return ctx, 2670 + 200 * rng.normal(size=125 * 119 * 61), rng.normal(size=10 * n)
+
+
+@pytest.mark.parametrize("line", ["below", "ahead"])
+@pytest.mark.parametrize("offset", OFFSETS)
+def test_station_next_to_a_mesh_line(line, offset):
+    ctx, mv, r = near_line(lambda m: LINES[line](m, offset))
+    K = KIND["joint"]
+    tiles, out = takes_tiles(ctx, K, mv)
+    assert not tiles
+    dm, ref = ctx.to_device(mv), ctx.alloc(out.size)
+    nat.check(ctx.lib.jgm_forward_noalloc(ctx.handle, K, nat.FP64, ctypes.c_void_p(dm.ptr),
+                                          ctypes.c_void_p(ref.ptr)))
+    ctx.synchronize()
+    ref = ref.to_host().reshape(-1, 10)
+    # the same corner terms, added in another order
+    assert np.all(np.abs(out.reshape(-1, 10) - ref) <= 1e-12 * np.max(np.abs(ref), axis=0))
+    ctx.profile_enable(True)
+    ctx.profile_reset()
+    ctx.adjoint(K, nat.FP64, None, r)
+    assert not any(name.startswith("tile") for name in ctx.profile())
+
+
+def test_stations_away_from_mesh_lines_take_the_tiles():
+    assert takes_tiles(*(lambda c, v, r: (c, KIND["joint"], v))(*near_line(None)))[0]
+    ctx, mv, _ = near_line(lambda m: LINES["below"](m, 0.05))
+    assert takes_tiles(ctx, KIND["joint"], mv)[0]
