@@ -171,9 +171,10 @@ __device__ inline void grad_absmax(const double* __restrict__ g, long n, int x, 
 
 // Adjoint at FC sample cells: block x < FC nsplit takes split x % nsplit of cell x / nsplit,
 // eight lanes per site, one for each corner of the cell,
-// g_c = 2 sum_s sum_m c_m(s) sum_corners sigma F_m (the gridded part; the background gradient
-// is exact in both paths); gs[cell nsplit + split].  The other nb blocks take the largest
-// |gradient| of their share.
+// g_c = 2 sum_s sum_corners sigma sum_m c_m(s) F_m (the gridded part; the background gradient
+// is exact in both paths); gs[cell nsplit + split].  The corners' difference is taken site by
+// site: corner sums over many sites would round at their own size, not at the gradient's.  The
+// other nb blocks take the largest |gradient| of their share.
 template <int MASK>
 __global__ __launch_bounds__(kBlock) void k_check_adjoint(
     const double* __restrict__ sx, const double* __restrict__ sy, const double* __restrict__ sz,
@@ -213,9 +214,12 @@ __global__ __launch_bounds__(kBlock) void k_check_adjoint(
     site_coefficients(rm, s, kind, fd, c7);
     double h = 0.0;
     for (int m = 0; m < 7; ++m) h = fma(c7[m], u[m], h);
-    acc += ((a + b + d) & 1) ? h : -h;
+    h = ((a + b + d) & 1) ? h : -h;
+#pragma unroll
+    for (int off = 1; off < 8; off *= 2) h += __shfl_xor(h, off, 64);
+    acc += h;
   }
-  const double g = block_sum(acc, red);
+  const double g = block_sum((threadIdx.x & 7) == 0 ? acc : 0.0, red);
   if (threadIdx.x == 0) gs[blockIdx.x] = 2.0 * g;
 }
 
