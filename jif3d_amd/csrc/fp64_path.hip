@@ -1727,7 +1727,7 @@ hipError_t launch_sensitivity_rows(jgm_context* ctx, int kind, size_t site0, siz
     const int tiles_k = (int)((n[2] + kTileK - 2) / (kTileK - 1));
     const int cells_k = (int)((n[2] + tiles_k - 1) / tiles_k);
     const long tiles = (long)tiles_i * tiles_j * tiles_k;
-    if (tiles < (1L << 31)) {
+    if (tiles * kTileThreads < (1L << 32)) {  // a launch dimension ends there
 #define JGM_ROWS(M, TWO)                                                                         \
   hipLaunchKernelGGL((k_sensitivity_row_tiles<M, TWO>), dim3((unsigned)tiles, (unsigned)nsites), \
                      dim3(kTileThreads), 0, ctx->stream, ctx->d_sx.as<double>(),                 \
