@@ -377,7 +377,7 @@ __device__ inline void store_row_entry(const double* u, int kind, FieldDir fd, l
 // Raw sensitivity rows for a range of sites (reference layout), one lane per
 // parameter column, per-cell 8-corner evaluation like the OMP imps: for meshes with gaps or
 // overlaps between cells, whose neighbours do not share corners (k_sensitivity_row_tiles
-// otherwise), and for background columns alone.
+// otherwise), for flat and thin ones (rows_take_bricks) and for background columns alone.
 template <int MASK>
 __global__ __launch_bounds__(kBlock) void k_sensitivity_rows(
     const double* __restrict__ sx, const double* __restrict__ sy, const double* __restrict__ sz,
@@ -1711,6 +1711,34 @@ hipError_t launch_adjoint_fp64_batch(jgm_context* ctx, int kind, size_t nsets,
   return hipSuccess;
 }
 
+// Whether rows take bricks of cells (as many as `bricks`, `columns` of columns of nk cells) or
+// every cell its own eight corners.  A brick's workgroup costs as much as 50 to 80 cells by
+// themselves before its first corner (filling the logarithm table, two barriers, idle threads), so
+// flat meshes and thin ones lose: 64 sites over 128 x 128 cells take, in ms (bricks, cells):
+//   one layer: gz 0.32, 0.06; FTG 0.61, 0.10; gz + FTG 0.32, 0.10; vertical gradient 0.92, 0.14;
+//     magnetization 0.58, 0.26
+//   four: gz 0.33, 0.19; FTG 0.66, 0.34; gz + FTG 0.35, 0.35; gradient 0.93, 0.49;
+//     magnetization 0.63, 0.88
+//   twelve: gz 0.46, 0.52; FTG 0.92, 0.89; gz + FTG 0.48, 0.92; gradient 1.34, 1.40;
+//     magnetization 0.90, 2.62
+//   64 x 64 x 32 cells: gz 0.21, 0.37; FTG 0.40, 0.62; gz + FTG 0.22, 0.64
+// Nanoseconds of either form for 64 sites, fitted to 20 meshes of 64 to 196608 cells.  The choice
+// is the geometry's and the kind's, not the number of sites', on which a row must not depend.
+bool rows_take_bricks(int kind, const size_t (&n)[3], long bricks, double columns, int nk) {
+  struct Cost {
+    double cell, brick, corner;
+  };
+  const Cost c = kind == JGM_KIND_SCALAR               ? Cost{0.040, 5.5, 0.0104}
+                 : kind == JGM_KIND_SCALAR_TENSOR      ? Cost{0.071, 5.6, 0.0106}
+                 : kind == JGM_KIND_MAGNETIC_GRADIENT  ? Cost{0.109, 5.5, 0.0096}
+                 : kind == JGM_KIND_MAGNETIZATION      ? Cost{0.205, 3.8, 0.0064}
+                                                       : Cost{0.069, 3.8, 0.0064};
+  constexpr double kSitesOfCall = 64.0, kCellsStart = 11000.0, kBricksStart = 4500.0;
+  const double cells = (double)n[0] * n[1] * n[2];
+  return kBricksStart + kSitesOfCall * bricks * (c.brick + c.corner * columns * (nk + 1)) <
+         kCellsStart + kSitesOfCall * cells * c.cell;
+}
+
 hipError_t launch_sensitivity_rows(jgm_context* ctx, int kind, size_t site0, size_t nsites,
                                    double* rows) {
   const long np = (long)nparams(ctx, kind);
@@ -1727,7 +1755,12 @@ hipError_t launch_sensitivity_rows(jgm_context* ctx, int kind, size_t site0, siz
     const int tiles_k = (int)((n[2] + kTileK - 2) / (kTileK - 1));
     const int cells_k = (int)((n[2] + tiles_k - 1) / tiles_k);
     const long tiles = (long)tiles_i * tiles_j * tiles_k;
-    if (tiles * kTileThreads < (1L << 32)) {  // a launch dimension ends there
+    // corner columns of a brick, on average
+    const double wj = (double)n[1] / tiles_j;
+    const double columns = edges ? 4.0 * wj : ((double)n[0] / tiles_i + 1.0) * (wj + 1.0);
+    if (tiles * kTileThreads < (1L << 32) &&  // a launch dimension ends there
+        rows_take_bricks(kind, n, tiles, columns, cells_k)) {
+      ProfScope ps(ctx, "sensitivity_rows_bricks_fp64");
 #define JGM_ROWS(M, TWO)                                                                         \
   hipLaunchKernelGGL((k_sensitivity_row_tiles<M, TWO>), dim3((unsigned)tiles, (unsigned)nsites), \
                      dim3(kTileThreads), 0, ctx->stream, ctx->d_sx.as<double>(),                 \
@@ -1748,6 +1781,7 @@ hipError_t launch_sensitivity_rows(jgm_context* ctx, int kind, size_t site0, siz
       return hipGetLastError();
     }
   }
+  ProfScope ps(ctx, "sensitivity_rows_cells_fp64");
   dim3 grid(blocks_for(np), (unsigned)nsites);
   const double* a[6] = {ctx->d_xlo.as<double>(), ctx->d_ylo.as<double>(), ctx->d_zlo.as<double>(),
                         ctx->d_xsz.as<double>(), ctx->d_ysz.as<double>(), ctx->d_zsz.as<double>()};
