@@ -1057,6 +1057,8 @@ bool choose(const jgm_context* ctx, bool tensor) {
   }
   const double ratio = tensor ? kRatio<kMaskAll> : kRatio<kMaskScalar>;
   const double tiles = (double)centre[0].size() * centre[1].size() * centre[2].size();
+  // a launch dimension ends at 2^32 threads: a workgroup per site, and one per tile
+  if (S * kBlock >= 1L << 32 || tiles * kNearThreads >= 0x1p32) return false;
   const long samples = std::min<long>(S, 16);
   double near = 0.0;
   for (long f = 0; f < samples; ++f) {

@@ -50,3 +50,21 @@ def test_rows_of_a_mesh_with_two_to_the_23_bricks(orc):
     rows.free()
     # offsets of whole metres are exact; eight logarithms and arctangents each
     assert max(errors) <= 1e-11 * largest
+
+
+def test_data_of_two_to_the_24_sites():
+    """A workgroup of 256 threads per site would be 2^32 threads."""
+    rng = np.random.default_rng(1)
+    dims, n = (100, 100, 6), 1 << 24
+    rho = 2670 + 200 * rng.normal(size=dims[0] * dims[1] * dims[2])
+    p = [rng.uniform(0, 2000, n), rng.uniform(0, 2000, n), -rng.uniform(3, 60, n)]
+    at = [0, 12345678, n - 1]
+    few, many = nat.Context(), nat.Context()
+    for ctx, sites in ((few, [v[at] for v in p]), (many, p)):
+        ctx.set_mesh(mesh(dims))
+        ctx.set_sites(*sites)
+    ref = few.forward(nat.KIND_SCALAR, nat.FP64, rho)
+    many.profile_enable(True)
+    out = many.forward(nat.KIND_SCALAR, nat.FP64, rho)
+    assert "forward_corners_fp64_gz" in many.profile()
+    assert np.max(np.abs(out[at] - ref)) <= 1e-12 * np.max(np.abs(ref))
