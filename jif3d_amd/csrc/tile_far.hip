@@ -1000,6 +1000,41 @@ TileGrid tile_grid(const jgm_context* ctx) {
   return g;
 }
 
+// How a geometry's sums are split.  None of it depends on the number of models, whose sums must
+// not either.
+struct TilePlan {
+  int ntiles, far_blocks, far_per, far_chunks;  // data, far: workgroups of sites, tiles a chunk
+  int near_splits;                              // data, near: rows of a site's sum
+  int adj_splits;                               // gradient, near: rows of a corner's sum
+};
+TilePlan tile_plan(const jgm_context* ctx) {
+  const TileGrid g = tile_grid(ctx);
+  const int S = (int)ctx->S;
+  TilePlan p;
+  p.ntiles = g.tx * g.ty * g.tz;
+  // chunks of tiles for about 16 waves per SIMD
+  p.far_blocks = (int)blocks_for((S + kSites - 1) / kSites);
+  const int want = std::max(1, std::min(p.ntiles, 16 * ctx->cu_count / p.far_blocks));
+  p.far_per = (p.ntiles + want - 1) / want;
+  p.far_chunks = (p.ntiles + p.far_per - 1) / p.far_per;
+  // a split per 1024 sites short of filling the CUs
+  p.near_splits = std::max(1, std::min(8, 2048 / S));
+  // for 8192 workgroups and more; beyond that a split only costs memory and the log tables again
+  // (gz, 512 x 512 x 64 cells and 1024 sites: near gradient 1.47 ms in four, 0.97 in one)
+  p.adj_splits = std::max(1, std::min(std::min(4, S / 256), 8192 / p.ntiles));
+  return p;
+}
+
+// Bytes of the buffers of a model's data and gradient: coefficients, corner weights and partial
+// sums; local expansions and corner sums.  (gz + FTG of 128 x 128 x 64 cells and 4096 sites: 54, 12
+// and 118 MB, 8 and 48 MB.)
+size_t tile_bytes(const jgm_context* ctx, const TilePlan& p, bool tensor) {
+  const size_t tile = (size_t)kNM * (tensor ? 12 : 2) + kTCorners + kRows +
+                      (size_t)p.adj_splits * kTCorners;
+  const size_t row = (size_t)(tensor ? 7 : 1) * ctx->S;
+  return sizeof(double) * (p.ntiles * tile + (p.far_chunks + p.near_splits + 1) * row);
+}
+
 HarmonicTable harmonic_table(const jgm_context* ctx) {
   const size_t* at = harmonic_block().at;
   const char* base = ctx->tile_far.table.as<const char>();
@@ -1087,7 +1122,8 @@ bool choose(const jgm_context* ctx, bool tensor) {
   const double closed = (double)ncorners(ctx) * term + (tensor ? 6.6e9 : 11.5e9) / (double)S;
   const double split = 1.9 * near * kTCorners * term + 3.0 * (tiles - near) * far_tile +
                        (3.0 * tiles * ends + (tensor ? 8.2e9 : 11.0e9)) / (double)S;
-  return split < closed;
+  // (one model's buffers take 42 KB a tile with the tensor: 64 GiB is 800 million cells)
+  return split < closed && tile_bytes(ctx, tile_plan(ctx), tensor) <= (size_t)64 << 30;
 }
 
 // The calls of a launch over nb in {1, 2, 4, 8} models, nb a template argument.
@@ -1109,13 +1145,8 @@ hipError_t forward_partials(jgm_context* ctx, int nb, const double* models, size
   TileFar& f = ctx->tile_far;
   hipStream_t st = ctx->stream;
   const TileGrid g = tile_grid(ctx);
-  const int ntiles = g.tx * g.ty * g.tz, S = (int)ctx->S;
-  // far: chunks of tiles for about 16 waves per SIMD; near: a split per 1024 sites short of
-  // filling the CUs; neither depends on the number of models, whose sums must not either
-  const int site_blocks = (int)blocks_for(S), far_blocks = (int)blocks_for((S + kSites - 1) / kSites);
-  const int want = std::max(1, std::min(ntiles, 16 * ctx->cu_count / far_blocks));
-  const int per = (ntiles + want - 1) / want, far_chunks = (ntiles + per - 1) / per;
-  const int splits = std::max(1, std::min(8, 2048 / S));
+  const TilePlan p = tile_plan(ctx);
+  const int ntiles = p.ntiles, S = (int)ctx->S, far_chunks = p.far_chunks, splits = p.near_splits;
   hipError_t e;
   if ((e = f.coefs.ensure(sizeof(double) * (size_t)nb * ntiles * kNM * 2 * NQ)) != hipSuccess ||
       (e = f.wt.ensure(sizeof(double) * (size_t)nb * ntiles * kTCorners)) != hipSuccess ||
@@ -1131,7 +1162,7 @@ hipError_t forward_partials(jgm_context* ctx, int nb, const double* models, size
     ProfScope ps(ctx, "tile_moments_fp64");
     hipLaunchKernelGGL(k_reference_density, dim3(nb), dim3(1024), 0, st, models, (long)model_ld,
                        (long)ncells(ctx), f.ref.as<double>());
-    hipLaunchKernelGGL((k_reference_box<MASK>), dim3(site_blocks), dim3(kBlock), 0, st, sx, sy, sz,
+    hipLaunchKernelGGL((k_reference_box<MASK>), dim3(blocks_for(S)), dim3(kBlock), 0, st, sx, sy, sz,
                        S, g, f.ref.as<const double>(), nb, part + (far_chunks + splits) * row, ld);
     hipLaunchKernelGGL((k_tile_moments<MASK>), dim3(ntiles, nb), dim3(kBlock), 0, st, g, ntiles,
                        models, (long)model_ld, f.ref.as<const double>(), harmonic_table(ctx),
@@ -1139,9 +1170,9 @@ hipError_t forward_partials(jgm_context* ctx, int nb, const double* models, size
   }
   {
     ProfScope ps(ctx, "tile_far_forward_fp64");
-    hipLaunchKernelGGL((k_tile_far_forward<MASK>), dim3(far_blocks, far_chunks, nb), dim3(kBlock),
+    hipLaunchKernelGGL((k_tile_far_forward<MASK>), dim3(p.far_blocks, far_chunks, nb), dim3(kBlock),
                        0, st, sx, sy, sz, S, f.geo.as<const double4>(),
-                       f.coefs.as<const double>(), ntiles, per, part, ld);
+                       f.coefs.as<const double>(), ntiles, p.far_per, part, ld);
   }
   {
     ProfScope ps(ctx, "tile_near_forward_fp64");
@@ -1162,8 +1193,8 @@ hipError_t adjoint_cells(jgm_context* ctx, int nb, const double* coef, double* g
   TileFar& f = ctx->tile_far;
   hipStream_t st = ctx->stream;
   const TileGrid g = tile_grid(ctx);
-  const int ntiles = g.tx * g.ty * g.tz, S = (int)ctx->S;
-  const int splits = std::max(1, std::min(4, S / 256));
+  const TilePlan p = tile_plan(ctx);
+  const int ntiles = p.ntiles, S = (int)ctx->S, splits = p.adj_splits;
   hipError_t e;
   if ((e = f.lam.ensure(sizeof(double) * (size_t)nb * ntiles * kRows)) != hipSuccess ||
       (e = ctx->hpart.ensure(sizeof(double) * (size_t)splits * nb * ntiles * kTCorners)) !=
@@ -1230,12 +1261,9 @@ hipError_t tile_far_prepare(jgm_context* ctx, int kind, bool* applies) {
   return hipSuccess;
 }
 
-// Models to a launch of the up to `left` that remain: the moments of one take 15 KB (gz + FTG) a
-// tile, so a mesh of 2^26 cells takes 2 GiB at a time, one of 2^29 cells in turn.
+// Models to a launch of the up to `left` that remain: as many as 2 GiB of their buffers hold.
 int tile_far_models(const jgm_context* ctx, int kind, size_t left) {
-  const TileGrid g = tile_grid(ctx);
-  const size_t one = sizeof(double) * kNM * (kind == JGM_KIND_SCALAR ? 2 : 12) * (size_t)g.tx *
-                     g.ty * g.tz;
+  const size_t one = tile_bytes(ctx, tile_plan(ctx), kind != JGM_KIND_SCALAR);
   int nb = left >= 8 ? 8 : left >= 4 ? 4 : left >= 2 ? 2 : 1;
   while (nb > 1 && nb * one > (size_t)2 << 30) nb /= 2;
   return nb;
