@@ -2,6 +2,7 @@
 // dispatch to the HIP kernels.  See include/jif3d_gravmag.h for the contract.
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
 #include <cerrno>
 #include <cmath>
 #include <cstdarg>
@@ -134,8 +135,8 @@ size_t data_per_site(const jgm_context* ctx, int kind) {
 
 // Host-memory form of a device entry point: copies the inputs to device buffers, runs `call`
 // on their device pointers, copies the outputs back and waits.  The device buffers are the
-// context's, kept between calls, up to kStageKept bytes a call (larger ones are given back when
-// the call ends); up to kStagePinned bytes the copies pass through the context's page-locked
+// context's, kept between calls, up to kStageKept bytes in all (a larger call's are given back when
+// it ends, and the kept ones before a call that would take them past it); up to kStagePinned bytes the copies pass through the context's page-locked
 // memory, with one wait at the end instead of one for each copy of pageable memory.  Data and
 // gradient of 4000 cells and 100 sites: 175 us with an allocation and pageable copies, 136 us.
 struct HostArg {
@@ -152,6 +153,13 @@ jgm_status run_staged(jgm_context* ctx, const char* where, const HostArg (&args)
   for (size_t a = 0; a < NA; ++a) total += sizeof(double) * args[a].n;
   hipError_t e = hipSuccess;
   const bool kept = total <= kStageKept;
+  if (kept) {
+    size_t held = 0;
+    for (size_t a = 0; a < sizeof(ctx->host_stage) / sizeof(ctx->host_stage[0]); ++a)
+      held += std::max(ctx->host_stage[a].bytes, a < NA ? sizeof(double) * args[a].n : 0);
+    if (held > kStageKept)  // every earlier call has waited for its copies
+      for (auto& b : ctx->host_stage) b.release();
+  }
   bool pinned = total <= kStagePinned;
   if (pinned && !ctx->host_pin &&
       hipHostMalloc(&ctx->host_pin, kStagePinned, hipHostMallocDefault) != hipSuccess) {

@@ -1,5 +1,5 @@
 """Device memory that a context keeps between calls: a batch's buffers stay within the stated 2 GiB
-however large the mesh."""
+however large the mesh, and the operands of host calls within 512 MB whichever calls came before."""
 import ctypes
 
 import numpy as np
@@ -40,3 +40,22 @@ def test_batch_on_a_large_mesh():
     one = ctx.alloc((n,))
     ctx.adjoint(nat.KIND_SCALAR, nat.FP64, None, ctx.to_device(r.to_host()[models - 1]), one)
     assert np.array_equal(one.to_host(), last)
+
+
+def test_operands_of_host_calls():
+    """A model of 480 MB in the one call, a gradient of 480 MB in the next."""
+    dims = (400, 400, 375)
+    n = dims[0] * dims[1] * dims[2]
+    ctx = nat.Context()
+    ctx.set_mesh(mesh(dims))
+    ctx.set_sites([3993.0], [4007.0], [-30.0])
+    model, grad = ctx.to_device(np.full(n, 2670.0)), ctx.alloc((n,))
+    data = ctx.alloc((1,))
+    ctx.forward(nat.KIND_SCALAR, nat.FP64, model, data)  # the kernels' own buffers
+    ctx.adjoint(nat.KIND_SCALAR, nat.FP64, None, data, grad)
+    before = free_bytes(ctx)
+    out = ctx.forward(nat.KIND_SCALAR, nat.FP64, np.full(n, 2670.0))
+    assert np.array_equal(out, data.to_host())
+    g = ctx.adjoint(nat.KIND_SCALAR, nat.FP64, None, out)
+    assert np.array_equal(g, grad.to_host())
+    assert before - free_bytes(ctx) <= (512 << 20) + SLACK
