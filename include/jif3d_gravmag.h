@@ -64,14 +64,14 @@ typedef enum jgm_kind {
   JGM_KIND_MAGNETIZATION = 6
 } jgm_kind;
 
-/* JGM_FP64: closed-form box terms in FP64 for every site-cell pair.  From 60000 cells and 64
- * sites (where it is faster for three models at a time; with the tensor, no site nearer a mesh line than
- * 2^-18 of the line's length ahead of it, where the closed form's logarithms are guarded or lost)
- * jgm_forward and jgm_adjoint of the scalar and scalar+tensor kinds sum tiles of 8 x 8 x 8 cells
- * farther than 3.95 (scalar) or 4.4 of their half-diagonals by FP64 solid-harmonic expansions of
- * degree 20.  What these leave out is within 1e-12 of each component's largest value over the
- * sites, whatever the densities, and below the closed form's own rounding of a few cells that far
- * away (1e-12 to 1e-11).
+/* JGM_FP64: closed-form box terms in FP64 for every site-cell pair.  jgm_forward and jgm_adjoint of
+ * the scalar and scalar+tensor kinds sum tiles of 8 x 8 x 8 cells farther than 3.95 (scalar) or 4.4
+ * of their half-diagonals by FP64 solid-harmonic expansions of degree 20, on meshes of 60000 cells
+ * and more with 64 sites and more, where that is faster for three models at a time and no site is
+ * nearer a mesh line (scalar kind: a horizontal one) than 2^-18 of the line's length ahead of it,
+ * where the closed form's logarithms are guarded or lost.  What the expansions leave out is within
+ * 1e-12 of each component's largest value over the sites, whatever the densities, and below the
+ * closed form's own rounding of a few cells that far away (1e-12 to 1e-11).
  * JGM_MIXED: FP64 closed form for cells inside each site's near box (every cell closer
  * than q0 of its own half-diagonals: the layers within their reach of the site, and along
  * x and y the largest reach of those layers), FP32 multipole of the prism about its centre

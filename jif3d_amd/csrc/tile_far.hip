@@ -1059,26 +1059,29 @@ bool choose(const jgm_context* ctx, bool tensor) {
   for (const auto* c : C)
     for (size_t i = 1; i < c->size(); ++i)
       if (!((*c)[i] > (*c)[i - 1])) return false;
-  // With the tensor, no station on or next to a mesh line.  Of the corners down a line at distance
+  // No station on or next to a mesh line.  Of the corners down a line at distance
   // rho, those at u < 0 along it have log(u + r), u + r = rho^2 / 2|u|, formed with an ulp of |u|:
   // guarded or a few ulps where rho is small, not the field but what the reference computes, and
   // tiles that are expanded would give the field instead.  At rho = 2^-18 of the farthest |u| (5 mm
-  // for 1.3 km) the argument keeps 15 bits and the closed form is the field with some noise.  (In
-  // gz a factor of rho stands before these logarithms.)
+  // for 1.3 km) the argument keeps 15 bits and the closed form is the field with some noise.
+  // gz has the logarithms of the horizontal lines only, times the offset from the line, without
+  // the guard: not a number on the line (as the reference's), 1e-8 of gz a micrometre beside it.
   const std::vector<double>* P[3] = {&ctx->hsx, &ctx->hsy, &ctx->hsz};
-  for (long s = 0; tensor && s < S; ++s) {
-    double plane2[3];  // squared distances to the nearest corner planes
-    for (int a = 0; a < 3; ++a) {
-      const double v = (*P[a])[s];
-      const auto up = std::lower_bound(C[a]->begin(), C[a]->end(), v);
-      double d = up != C[a]->end() ? *up - v : HUGE_VAL;
-      if (up != C[a]->begin()) d = std::min(d, v - up[-1]);
-      plane2[a] = d * d;
-    }
-    for (int a = 0; a < 3; ++a) {
-      const double u = std::max(0.0, C[a]->back() - (*P[a])[s]);
-      if (plane2[(a + 1) % 3] + plane2[(a + 2) % 3] <= 0x1p-36 * u * u) return false;
-    }
+  auto plane = [&](int a, long s) {  // distance to the nearest corner plane
+    const double v = (*P[a])[s];
+    const auto up = std::lower_bound(C[a]->begin(), C[a]->end(), v);
+    const double above = up != C[a]->end() ? *up - v : HUGE_VAL;
+    return up != C[a]->begin() ? std::min(above, v - up[-1]) : above;
+  };
+  auto ahead = [&](int a, long s) { return std::max(0.0, C[a]->back() - (*P[a])[s]); };
+  for (long s = 0; s < S; ++s) {
+    const double ux = ahead(0, s), uy = ahead(1, s), dz = plane(2, s);
+    if (!tensor && dz > 0x1p-18 * std::max(ux, uy)) continue;
+    const double dx = plane(0, s), dy = plane(1, s);
+    if (dy * dy + dz * dz <= 0x1p-36 * ux * ux || dx * dx + dz * dz <= 0x1p-36 * uy * uy)
+      return false;
+    const double uz = tensor ? ahead(2, s) : 0.0;
+    if (tensor && dx * dx + dy * dy <= 0x1p-36 * uz * uz) return false;
   }
   // near tiles of a sample of stations
   std::vector<double> centre[3], half2[3];

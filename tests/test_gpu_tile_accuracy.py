@@ -161,3 +161,23 @@ def test_stations_away_from_mesh_lines_take_the_tiles():
     assert takes_tiles(*(lambda c, v, r: (c, KIND["joint"], v))(*near_line(None)))[0]
     ctx, mv, _ = near_line(lambda m: LINES["below"](m, 0.05))
     assert takes_tiles(ctx, KIND["joint"], mv)[0]
+
+
+# gz has the logarithms of the horizontal lines only, unguarded, behind the offset from the line
+@pytest.mark.parametrize("offset", OFFSETS)
+def test_gz_next_to_a_mesh_line(offset):
+    ctx, mv, r = near_line(lambda m: LINES["ahead"](m, offset))
+    K = KIND["gz"]
+    tiles, out = takes_tiles(ctx, K, mv)
+    assert not tiles
+    dm, ref = ctx.to_device(mv), ctx.alloc(out.size)
+    nat.check(ctx.lib.jgm_forward_noalloc(ctx.handle, K, nat.FP64, ctypes.c_void_p(dm.ptr),
+                                          ctypes.c_void_p(ref.ptr)))
+    ctx.synchronize()
+    ref = ref.to_host()
+    ok = np.isfinite(ref)
+    assert np.array_equal(ok, np.isfinite(out)) and np.all(np.delete(ok, 5))
+    worst = np.max(np.abs(out - ref)[ok])
+    assert worst <= 1e-12 * np.max(np.abs(ref[ok]))
+    above, mv, _ = near_line(lambda m: LINES["below"](m, offset))
+    assert takes_tiles(above, K, mv)[0]
