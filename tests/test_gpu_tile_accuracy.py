@@ -181,3 +181,58 @@ def test_gz_next_to_a_mesh_line(offset):
     assert worst <= 1e-12 * np.max(np.abs(ref[ok]))
     above, mv, _ = near_line(lambda m: LINES["below"](m, offset))
     assert takes_tiles(above, K, mv)[0]
+
+
+# Every station, not the worst few: gz + FTG data against the closed form, off-diagonal components
+# within the rounding that the closed form's logarithms have at that very station; an axis that
+# leaves one cell for its last tile, few stations, and one context through several
+# meshes and surveys.
+def survey(ctx, dims, nsites, seed):
+    from test_gpu_tile_far import rounding
+    rng = np.random.default_rng(seed)
+    m = ThreeDGravityModel()
+    m.SetMeshSize(*dims)
+    m.SetXCellSizes(np.full(dims[0], 20.0))
+    m.SetYCellSizes(np.full(dims[1], 20.0))
+    m.SetZCellSizes(np.full(dims[2], 15.0))
+    m.shape = dims
+    d = TensorGravityData()
+    d.SetMeasurementPoints(rng.uniform(-100, 20.0 * dims[0] + 100, nsites),
+                           rng.uniform(-100, 20.0 * dims[1] + 100, nsites),
+                           -rng.uniform(3, 60, nsites))
+    ctx.configure(m, d)
+    rho = 2670 + 200 * rng.normal(size=dims[0] * dims[1] * dims[2])
+    for kind, k in (("gz", 1), ("joint", 10)):
+        K = KIND[kind]
+        tiles, out = takes_tiles(ctx, K, rho)
+        dm, ref = ctx.to_device(rho), ctx.alloc(out.size)
+        nat.check(ctx.lib.jgm_forward_noalloc(ctx.handle, K, nat.FP64, ctypes.c_void_p(dm.ptr),
+                                              ctypes.c_void_p(ref.ptr)))
+        ctx.synchronize()
+        out, ref = out.reshape(-1, k), ref.to_host().reshape(-1, k)
+        for c in range(k):
+            tol = (1e-12 if c == 0 else 1e-11) * np.max(np.abs(ref[:, c]))
+            error = np.abs(out[:, c] - ref[:, c])
+            axis = {2: 2, 4: 2, 3: 1, 7: 1, 6: 0, 8: 0}.get(c)  # xy, xz, yz
+            for s in np.nonzero(error > tol)[0]:
+                assert axis is not None, (kind, c, s, error[s], tol)
+                assert error[s] <= tol + rounding(m, d, rho, s, axis), (kind, c, s, error[s])
+        # the gradient is the data's transpose
+        r = rng.normal(size=nsites * k)
+        if k == 10:
+            r = (r.reshape(-1, 10) * ([1.0] + [500.0] * 9)).ravel()
+        g = ctx.adjoint(K, nat.FP64, None, r)
+        left, right = 2.0 * float(out.ravel() @ r), float(g @ rho)
+        assert abs(left - right) <= 1e-10 * float(np.abs(out.ravel()) @ np.abs(r))
+        yield tiles
+
+
+def test_every_station_and_a_reused_context():
+    ctx = nat.Context()
+    assert list(survey(ctx, (97, 105, 65), 150, 1)) == [True, True]
+    assert list(survey(ctx, (128, 113, 49), 333, 2)) == [True, True]
+    assert list(survey(ctx, (30, 30, 20), 100, 3)) == [False, False]
+    assert list(survey(ctx, (97, 105, 65), 200, 4)) == [True, True]
+    assert list(survey(ctx, (128, 128, 64), 100, 5))[0]
+    list(survey(ctx, (128, 128, 16), 64, 5))  # on the line of stations, whichever is taken
+    assert list(survey(ctx, (128, 128, 16), 63, 6)) == [False, False]
