@@ -177,9 +177,11 @@ jgm_status jgm_forward_host(jgm_context *ctx, jgm_kind kind, jgm_precision prec,
  * No counterpart in the reference.  It calls no hipMalloc / hipFree and no allocating
  * library routine: its working memory (background table, corner weights, partial sums)
  * is one static device array of JGM_NOALLOC_SCRATCH_BYTES per GPU, reserved when the
- * library is loaded and held until the process ends.  Same arguments and results as
- * jgm_forward with JGM_FP64 (sums grouped into fewer chunks, so results agree to FP64
- * rounding, not bit for bit); JGM_MIXED, JGM_KIND_MAGNETIC_GRADIENT and
+ * library is loaded and held until the process ends.  Same arguments as
+ * jgm_forward with JGM_FP64, and its results to FP64 rounding, not bit for bit: it takes the
+ * closed form on every mesh, its sums grouped into fewer chunks (so do jgm_sensitivity_rows and
+ * the stored J; where jgm_forward takes expansions, the two differ by the closed form's rounding
+ * and by what the expansions leave out, see JGM_FP64); JGM_MIXED, JGM_KIND_MAGNETIC_GRADIENT and
  * JGM_KIND_MAGNETIZATION return JGM_ERR_UNSUPPORTED, and so does a problem whose
  * (mesh corners + 7 nsites nlayers + components nsites + nlayers) doubles exceed the
  * scratch.  Unlike jgm_forward it keeps no raw data for a later jgm_adjoint.  The mesh,

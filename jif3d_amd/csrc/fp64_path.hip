@@ -449,10 +449,12 @@ __global__ __launch_bounds__(kBlock) void k_sensitivity_rows(
 //    instead of 8).
 //  * the tensor alone and the vertical gradient (which carries the z column at the site and 1 m
 //    below): 7 columns along y, each with its own four corner edges, shared down the column (4.1
-//    per cell).  Down a line of corners that passes near the site log(u + r) turns an ulp of r
-//    into up to 1e-7 of a row's rms, and these rows have no larger component to hide it: the four
-//    edges of a column round r^2 each in its own way (edge_r2), as a cell by itself does, and the
-//    entries keep that rounding.
+//    per cell), whose r^2 round each in its own way (edge_r2), as a cell by itself does.
+// Down a line of corners that passes near the site log(u + r) turns an ulp of r into up to 1e-7 of a
+// row's rms.  Both forms, and cells by themselves, are equally far from the exact rows (against
+// extended precision, 40 x 40 x 24 cells, off-diagonal rows: 3.1e-11 of their rms on average and
+// 2.9e-8 at most with r rounded per cell, 3.2e-11 and 2.9e-8 with shared corners), but not with the
+// same noise: the second form's rows are the cells' own, the first form's move by it.
 // 512 threads and at most 63 KB of LDS put two workgroups on a CU.  Rows of 64 sites over
 // 64 x 64 x 32 cells: gz + FTG 0.26 ms (eight evaluations per cell 0.68), FTG 0.40 ms (0.61); the
 // 604 MB of the FTG rows take 0.12 ms at a copy's rate.

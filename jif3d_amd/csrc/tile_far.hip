@@ -346,13 +346,12 @@ __global__ __launch_bounds__(kBlock) void k_tile_moments(TileGrid g, int ntiles,
 
 // Data, far tiles: a lane has kSites sites (64 apart), a workgroup of four waves walks a chunk of
 // tiles.  The tile's coefficients (26 KB, gz 4 KB) go through LDS, the next tile's on their way
-// behind the sums (through 100 bytes of scratch a lane for gz + FTG, whose sums leave no
-// registers): as scalar loads, which the scalar cache does not hold, their latency took twice the
-// rest (2048 tiles and 4096 sites, gz + FTG, degree 16: 0.83 ms, 1.90 ms with scalar loads, 0.62 ms
-// is the VALU's; degree 20: 1.25 ms).  Orders m outermost, so a lane holds one h recurrence and the
-// 2 NQ sums of the order per site: 3 FP64 operations per (n, m) for h and 12 (gz: 2) for the sums.
-// Sums in the corner sums' signs and components: partial[model ld + (chunk NC + m) S + s]; grid:
-// z = models.
+// through 128 bytes of scratch a lane for gz + FTG: as scalar loads, which the scalar cache does
+// not hold, their latency took twice the rest (2048 tiles and 4096 sites, gz + FTG, degree 16: 0.83
+// ms, 1.90 ms with scalar loads, 0.62 ms is the VALU's; degree 20: 1.25 ms).  Orders m outermost,
+// so a lane holds one h recurrence and the 2 NQ sums of the order per site: 3 FP64 operations per
+// (n, m) for h and 12 (gz: 2) for the sums.  Sums in the corner sums' signs and components:
+// partial[model ld + (chunk NC + m) S + s]; grid: z = models.
 constexpr int kSites = 2;
 // entry of (n, m) in a tile's coefficients
 __host__ __device__ constexpr int entry_nm(int n, int m) {
